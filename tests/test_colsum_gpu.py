@@ -241,3 +241,20 @@ def test_select_windows(torch_gpu, case):
     if case == "sorted":  # the per-entry kernels (64-bit indices) agree
         got64 = _select_raw(indptr, idx, val, m, cols, torch, bits=64)
         assert all(np.array_equal(a, b) for a, b in zip(got, got64))
+
+
+@pytest.mark.parametrize("n,m,per_row", [(1, 70000, 3000), (124, 65536, 50), (125, 98305, 50), (500, 6000001, 200),
+                                         (4097, 200001, 60)])
+@pytest.mark.parametrize("bits", [32, 64])
+def test_column_segments(torch_gpu, n, m, per_row, bits):
+    """Few rows over many windows: the columns are cut into segments (one to all windows), rows
+    into blocks of 124 and more; rows out of order in one place still reach the per-entry path."""
+    indptr, idx, val = _random_csr(n, m, per_row, seed=n + m, vmax=1000)
+    status = []
+    assert np.array_equal(_sums(indptr, idx, val, m, bits, torch_gpu, status), _expected(idx, val, m))
+    assert status == [0]
+    r = int(np.argmax(np.diff(indptr)))
+    a, b = indptr[r], indptr[r + 1]
+    idx[a:b] = idx[a:b][::-1].copy()
+    assert np.array_equal(_sums(indptr, idx, val, m, bits, torch_gpu, status), _expected(idx, val, m))
+    assert status == [0, 1]
