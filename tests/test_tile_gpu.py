@@ -318,3 +318,47 @@ def test_sort_rows_entry_and_unsorted_status(torch_gpu):
     _lib.check(L.snapgpu_tile_count(fr.cell_ptr.data_ptr(), fr.pos.data_ptr(), fr.values.data_ptr(), len(cells),
                                     tab.data_ptr(), 1, 500, 2, 0, 0xFFFFFFFF, rows.data_ptr(), 0,
                                     status.data_ptr(), ctypes.byref(level), _lib.stream_ptr()))
+
+
+def _segment_cells(rng, cs):
+    """Rows around the segment kernel's edges (256 fragments per segment, 4 per lane): lengths on
+    both sides of whole segments; piles of one bin longer than a segment; fragments that reach
+    over a segment's end by 1 to 31 bins of 100 bases, over filtered and excluded fragments too."""
+    starts = dict(zip(cs, np.cumsum([0] + list(cs.values()))))
+    cells = []
+    for n in (0, 1, 3, 4, 255, 256, 257, 259, 511, 512, 513, 1030):
+        pos = np.sort(rng.integers(0, cs["chr1"] - 4000, n))
+        cells.append([(int(a), int(b)) for a, b in zip(pos, rng.integers(1, 3100, n))])
+    cells.append([(5000 + i // 200, 1 + (i * 37) % 3100) for i in range(900)])      # one pile
+    cells.append([(100 * i, 3101 if i % 5 else 20) for i in range(600)])            # spans of 31 bins
+    cells.append([(40 * i, 1500) for i in range(254)] + [(254 * 40 + i, 30) for i in range(300)])
+    mixed = [(int(a), 200) for a in np.sort(rng.integers(0, cs["chr1"] - 300, 250))]
+    mixed += [(starts["chrM"] + 3 * i, 50) for i in range(300)]                     # excluded
+    mixed += [(starts["chrX"] + 2 * i, 150 + i % 900) for i in range(700)]
+    cells.append(mixed)
+    return cells
+
+
+@pytest.mark.parametrize("n_cells", [16, 1023, 1024, 8191, 8192])
+@pytest.mark.parametrize("strategy", ["insertion", "fragment", "paired-insertion", "single"])
+def test_segments(torch_gpu, strategy, n_cells):
+    """16, 4 and 1 waves per cell (the cell counts lie on both sides of the rule)."""
+    rng = np.random.default_rng(n_cells)
+    cs = {"chr1": 70000, "chrM": 2000, "chrX": 20000}
+    cells = _segment_cells(rng, cs)
+    while len(cells) < n_cells:
+        pos = np.sort(rng.integers(0, 59000, int(rng.integers(0, 40))))
+        cells.append([(int(a), int(rng.integers(1, 900))) for a in pos])
+    for lo, hi in ((None, None), (40, 2000)):
+        m, _, (cp, pos, ln) = _tile(torch_gpu, cells, cs, 100, ["chrM"], lo, hi, strategy)
+        _same(m, otile.tile_matrix(cp, pos, ln, cs, 100, ["chrM"], lo, hi, strategy))
+
+
+@pytest.mark.parametrize("length", [3101, 3201, 3301])
+def test_segments_hand_over_long_fragments(torch_gpu, length):
+    """A fragment over more than 32 bins sends the call to the tile kernel; same matrix."""
+    cs = {"chr1": 60000}
+    cells = [[(50 * i, 120) for i in range(700)], [(90, 300), (99, length), (4000, 10)]]
+    for strategy in ("insertion", "paired-insertion", "fragment"):
+        m, _, (cp, pos, ln) = _tile(torch_gpu, cells, cs, 100, [], None, None, strategy)
+        _same(m, otile.tile_matrix(cp, pos, ln, cs, 100, [], None, None, strategy))
