@@ -164,3 +164,24 @@ def test_knn_dropin_with_50_components(torch_gpu):
     _check(ad.obsp["distances"], X, 150)
     g = snap.pp.knn(ad, n_neighbors=30, use_dims=45, inplace=False)
     _check(g, np.ascontiguousarray(X[:, :45]), 30)
+
+
+@pytest.mark.parametrize("n,d,k", [(129, 3, 25), (129, 3, 26), (2777, 8, 25), (2777, 8, 26), (640, 29, 1),
+                                   (15, 2, 14), (6000, 2, 25)])
+def test_candidate_lists(torch_gpu, n, d, k):
+    """Both sides of the rule for the candidates per lane (16 up to k = 25, else 32), with chunks
+    that are not full; few rows may need the second tier (more than 16 of the nearest in one
+    stripe: one query in 50,000 at k = 25)."""
+    from snapatac2_amd.pp._knn import nearest_neighbour_graph
+    X = clustered(n, d, n_clusters=3, seed=n + k)
+    g, st = nearest_neighbour_graph(X, k, return_stats=True)
+    _check(g, X, k)
+    assert st["exact_scan_rows"] == 0 or n < 4 * k
+
+
+def test_candidates_far_from_the_centre(torch_gpu):
+    """Values from 1e-3 to 1e12 in one matrix: the padding rows' score stays below the real ones'."""
+    from snapatac2_amd.pp._knn import nearest_neighbour_graph
+    rng = np.random.default_rng(5)
+    X = rng.standard_normal((900, 6)) * 10.0 ** rng.integers(-3, 13, 900)[:, None]
+    _check(nearest_neighbour_graph(X, 20), X, 20)
