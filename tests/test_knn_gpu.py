@@ -185,3 +185,32 @@ def test_candidates_far_from_the_centre(torch_gpu):
     rng = np.random.default_rng(5)
     X = rng.standard_normal((900, 6)) * 10.0 ** rng.integers(-3, 13, 900)[:, None]
     _check(nearest_neighbour_graph(X, 20), X, 20)
+
+
+@pytest.mark.parametrize("kind,n,d", [("clusters", 16383, 30), ("clusters", 16385, 30), ("clusters", 33001, 7),
+                                      ("one cluster", 25000, 30), ("line", 40000, 1), ("duplicates", 20001, 4),
+                                      ("constant", 16400, 3), ("scales", 30000, 5)])
+def test_cells(torch_gpu, kind, n, d):
+    """From 16,384 rows on (128 leaves) the rows are ordered by cells and chunks are skipped by
+    the planes between them: the graph of a run that skips nothing, and the oracle's rows."""
+    from snapatac2_amd.pp._knn import nearest_neighbour_graph
+    rng = np.random.default_rng(n)
+    k = 30
+    X = {"clusters": lambda: clustered(n, d, seed=n),
+         "one cluster": lambda: rng.standard_normal((n, d)),
+         "line": lambda: rng.random((n, 1)),
+         "duplicates": lambda: rng.integers(0, 9, (n, d)).astype(np.float64),
+         "constant": lambda: np.full((n, d), 0.25),
+         "scales": lambda: rng.standard_normal((n, d)) * 10.0 ** rng.integers(-4, 5, n)[:, None]}[kind]()
+    g = nearest_neighbour_graph(X, k)
+    full = nearest_neighbour_graph(X, k, prune=False)
+    assert np.array_equal(g.indices, full.indices) and np.array_equal(g.data, full.data)
+    rows = rng.choice(n, 300, replace=False)
+    d2 = np.zeros((300, n))
+    for c in range(d):  # the reference's order and rounding
+        d2 += (X[rows, c][:, None] - X[:, c][None]) ** 2
+    d2[np.arange(300), rows] = np.inf
+    for i, r in enumerate(rows):
+        near = np.sort(np.argsort(d2[i], kind="stable")[:k])
+        assert np.array_equal(g.indices[r * k:(r + 1) * k], near)
+        assert np.array_equal(g.data[r * k:(r + 1) * k], np.sqrt(d2[i, near]))
