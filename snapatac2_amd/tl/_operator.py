@@ -150,14 +150,14 @@ class SpectralOperator:
         if layout in ("mixed", "window"):
             fits = True
             try:
-                self.window_csr = self._build_window(X.indptr, X.indices, X.data, n, m, X.nnz)
+                # the default: too few window workgroups to fill the device and nothing is built
+                need = MIXED_MIN_BLOCKS if layout == "mixed" and chosen else 0
+                self.window_csr = self._build_window(X.indptr, X.indices, X.data, n, m, X.nnz, need)
                 if layout == "window":
                     self.window_csc = self._build_window(self.colptr, self.rowidx, self.cval, m, n, X.nnz)
             except _lib.CapacityError:
                 fits = False  # counts >= 256 or too many windows
-            if fits and layout == "mixed" and chosen and self.window_csr.n_blocks < MIXED_MIN_BLOCKS:
-                fits = False  # the default: too few window workgroups to fill the device
-            if not fits:  # the panel layout takes them
+            if not fits or self.window_csr is None:  # the panel layout takes them
                 self._panel_keep = []
                 self.window_csr = self.window_csc = None
                 layout = self.layout = "panel"
@@ -218,8 +218,9 @@ class SpectralOperator:
                                 rp_ptr.data_ptr(), rp_ids.data_ptr(), K.value, nrows, dense_rows,
                                 packed.value, self.value_type)
 
-    def _build_window(self, ptr, idx, val, nrows: int, dense_rows: int, nnz: int):
-        """Window layout of one storage direction (see snapgpu_window_plan/build)."""
+    def _build_window(self, ptr, idx, val, nrows: int, dense_rows: int, nnz: int, min_blocks: int = 0):
+        """Window layout of one storage direction (see snapgpu_window_plan/build), None
+        when the plan has fewer than min_blocks workgroups."""
         torch = self.torch
         L = _lib.lib()
         dev = ptr.device
@@ -235,6 +236,8 @@ class SpectralOperator:
                                          h_row_slot.ctypes.data, st))
         del ws
         nb = nb.value
+        if nb < min_blocks:
+            return None
         block_row = torch.from_numpy(h_block_row[:nb + 1]).to(dev)
         row_slot = torch.from_numpy(h_row_slot.view(np.int32)).to(dev)
         nw = int(L.snapgpu_window_count(dense_rows))
