@@ -47,22 +47,26 @@ using spectral::scale_in_kernel;
 constexpr int64_t kPanel = SNAPGPU_PANEL_ROWS;  // dense rows per panel (<= 32768: 15-bit column)
 constexpr int64_t kChunk = SNAPGPU_PANEL_CHUNK;  // entries per group-chunk at most (aligned to pair starts)
 constexpr int64_t kMinChunk = 256;               // and at least
-constexpr int64_t kChunkTarget = 32768;          // group-chunks that fill the chip: 4 per wave, 32 waves per CU
+constexpr int64_t kChunkTarget = 65536;          // group-chunks that fill the chip twice: 4 per wave, 32 waves per CU
 #ifndef SNAPGPU_PANEL_INFLIGHT
 #define SNAPGPU_PANEL_INFLIGHT 8
 #endif
 constexpr int kInflight = SNAPGPU_PANEL_INFLIGHT;  // gathers in flight per lane
 #ifndef SNAPGPU_PANEL_INFLIGHT16
-#define SNAPGPU_PANEL_INFLIGHT16 8
+#define SNAPGPU_PANEL_INFLIGHT16 16
 #endif
-constexpr int kInflight16 = SNAPGPU_PANEL_INFLIGHT16;  // the same, 16-column packed-8 product
+// the same, 16-column packed-8 product: 16 against 8, per application of 3.9M entries
+// 117 and 142 us, of 130M 1.97 and 2.00 ms, of 820M (with windows) 13.53 and 13.64 ms
+constexpr int kInflight16 = SNAPGPU_PANEL_INFLIGHT16;
 static_assert(kPanel <= 32768, "the packed entry holds a 15-bit column");
 
 // Entries per group-chunk. A group streams its chunk alone, so a small matrix in
 // chunks of kChunk leaves most CUs idle and the others waiting for gathers: below
 // kChunkTarget chunks they get shorter (3.8M entries, 16 columns: 244 -> 59 us
-// per product), down to 4 batches of 64 entries. Sums do not depend on it: a pair
-// lies in one chunk whatever the size.
+// per product), down to 4 batches of 64 entries. Twice what fits the chip also
+// evens out the last groups (130M entries: 2.07 ms per application of 32,768
+// chunks, 1.97 of 65,536, 1.95 of 131,072, where 26M entries lose 3%). A pair lies in
+// one chunk whatever the size.
 static int64_t chunk_entries(int64_t nnz) {
   return std::min(kChunk, std::max(kMinChunk, ceil_div(ceil_div(nnz, kChunkTarget), 64) * 64));
 }
@@ -220,8 +224,15 @@ __global__ void chunk_kernel(const int64_t* __restrict__ pstart, const int64_t* 
 // group-chunk wave * G + g: 4 * BW entries per batch, one coalesced dword per
 // lane per quarter; entry j of the batch is broadcast to the group from lane
 // j % BW, register j / BW. Gathers are issued kInflight at a time. A pair's first entry
-// carries a flag: the running sum of the previous pair is stored and reset.
+// carries a flag: the running sum of the previous pair is stored and reset. The sum
+// is taken in blocks of kSumBlock entries of the batch, added one after the other, so
+// that its rounding grows with the blocks and not with the entries of a pair (a
+// feature's whole column where the cells fit one panel): relative error of the weight
+// adjoint of 20,000 cells x 100,000 features 1.25e-6 in one run of entries, 3.6e-7 so
 // ---------------------------------------------------------------------------
+constexpr int kSumBlock = 16;
+static_assert(kSumBlock % kInflight == 0 && kInflight16 == kSumBlock, "a step of gathers is (part of) one block");
+
 template <int MODE, bool FV>
 __device__ __forceinline__ float entry_value(uint32_t e, uint32_t v) {
   if (MODE == 2) return (float)((e >> 24) & 0x7Fu);
@@ -267,7 +278,7 @@ __global__ void __launch_bounds__(256) product_kernel(const uint32_t* __restrict
     db = dense + (int64_t)cpanel[chunk] * kPanel * BW;
   }
   bool have = false;  // a pair is open (its first entry was seen)
-  float acc = 0.f;
+  float acc = 0.f, sum = 0.f;  // the open pair's finished blocks, and the block at hand
   while (__ballot(pos < end) != 0) {
     uint32_t e[4], v[4];
 #pragma unroll
@@ -291,11 +302,16 @@ __global__ void __launch_bounds__(256) product_kernel(const uint32_t* __restrict
 #pragma unroll
       for (int u = 0; u < kInflight; ++u) {
         if (ej[u] & kFirst) {
-          if (have) partial[k++ * BW + c] = acc;
+          if (have) partial[k++ * BW + c] = acc + sum;
           have = true;
           acc = 0.f;
+          sum = 0.f;
         }
-        acc = fmaf(entry_value<MODE, FV>(ej[u], vj[u]), z[u], acc);
+        sum = fmaf(entry_value<MODE, FV>(ej[u], vj[u]), z[u], sum);
+        if ((j0 + u + 1) % kSumBlock == 0) {
+          acc += sum;
+          sum = 0.f;
+        }
       }
     }
     pos += NB;
@@ -331,7 +347,7 @@ __device__ __forceinline__ void bcast_entries(uint32_t (&v)[sizeof...(U)], const
   ((v[U] = row_bcast<(J0 + U) % 16>(e[(J0 + U) / 16])), ...);
 }
 
-// INF entries of the batch, starting at J0. A first-of-pair entry carries
+// INF entries of the batch, one block of the sum, starting at J0. A first-of-pair entry carries
 // count + 128 in byte 3: its pair's sum starts at -128 * z, so that
 // fma(count + 128, z, -128 * z) rounds (count + 128) * z - 128 * z = count * z
 // exactly as the generic kernel's fma(count, z, 0) does (-128 * z is exact).
@@ -355,20 +371,23 @@ __device__ __forceinline__ void gather16_step(const uint32_t (&e)[4], const char
   uint32_t any = 0;
 #pragma unroll
   for (int u = 0; u < INF; ++u) any |= v[u];
+  float sum = 0.f;  // of this block of INF entries
   if (__builtin_amdgcn_ballot_w64((int32_t)any < 0) == 0) {
 #pragma unroll
-    for (int u = 0; u < INF; ++u) acc = fmaf((float)(v[u] >> 24), z[u], acc);
+    for (int u = 0; u < INF; ++u) sum = fmaf((float)(v[u] >> 24), z[u], sum);
   } else {
 #pragma unroll
     for (int u = 0; u < INF; ++u) {
       if ((int32_t)v[u] < 0) {
-        if (have) partial[(int64_t)k++ * 16 + c] = acc;
+        if (have) partial[(int64_t)k++ * 16 + c] = acc + sum;
         have = true;
-        acc = -128.f * z[u];
+        acc = 0.f;
+        sum = -128.f * z[u];
       }
-      acc = fmaf((float)(v[u] >> 24), z[u], acc);
+      sum = fmaf((float)(v[u] >> 24), z[u], sum);
     }
   }
+  acc += sum;
 }
 
 template <int INF, bool TAIL, int... S>
@@ -449,20 +468,22 @@ __global__ void __launch_bounds__(256) reduce_kernel(const int64_t* __restrict__
   const int64_t row = t / BW;
   const int c = (int)(t % BW);
   if (row >= nrows) return;
-  // pairs in panel order; four loads in flight, added in the same order
+  // pairs in panel order; four loads in flight, added in the same order, in FP64 (the
+  // kernel waits for the loads): one rounding to FP32 per row instead of one per pair
   const int64_t i0 = rp_ptr[row], i1 = rp_ptr[row + 1];
-  float acc = 0.f;
+  double sum = 0.0;
   int64_t i = i0;
   for (; i + 4 <= i1; i += 4) {
     const int32_t p0 = rp_ids[i], p1 = rp_ids[i + 1], p2 = rp_ids[i + 2], p3 = rp_ids[i + 3];
     const float a0 = partial[(int64_t)p0 * BW + c], a1 = partial[(int64_t)p1 * BW + c];
     const float a2 = partial[(int64_t)p2 * BW + c], a3 = partial[(int64_t)p3 * BW + c];
-    acc += a0;
-    acc += a1;
-    acc += a2;
-    acc += a3;
+    sum += (double)a0;
+    sum += (double)a1;
+    sum += (double)a2;
+    sum += (double)a3;
   }
-  for (; i < i1; ++i) acc += partial[(int64_t)rp_ids[i] * BW + c];
+  for (; i < i1; ++i) sum += (double)partial[(int64_t)rp_ids[i] * BW + c];
+  const float acc = (float)sum;
   if (EPI == 0) {
     out32[row * BW + c] = scale ? acc * scale[row] : acc;
   } else if (c < b) {
@@ -504,6 +525,11 @@ static void launch_product(const snapgpu_panel_layout& L, const float* dense, fl
 void product16_scaled(const snapgpu_panel_layout& L, const float* dense, float* partial, const float* scale,
                       float* out, hipStream_t st) {
   launch_product<16, 0>(L, dense, partial, scale, out, nullptr, 0, nullptr, nullptr, 0, 16, st);
+}
+
+void product32_scaled(const snapgpu_panel_layout& L, const float* dense, float* partial, const float* scale,
+                      float* out, hipStream_t st) {
+  launch_product<32, 0>(L, dense, partial, scale, out, nullptr, 0, nullptr, nullptr, 0, 32, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -820,7 +846,11 @@ int snapgpu_spectral_apply_panel(const snapgpu_panel_layout* csr, const snapgpu_
   scale_in_kernel<BW><<<(unsigned)ceil_div(n * BW, 256), 256, 0, st>>>(d_V, ldv, n, b, d_r32, Vs);         \
   launch_product<BW, 0>(*csc, Vs, part, d_w2, Z, nullptr, 0, nullptr, nullptr, 0, b, st);                 \
   launch_product<BW, 1>(*csr, Z, part, d_r32, nullptr, d_V, ldv, d_dinv, d_Y, ldy, b, st);
-  if (b <= 8) {
+  // 16-column rows for b <= 8 too where both directions take product16_kernel: half of a
+  // gathered row is padding, but the 8-column product spends more on instructions
+  // (130M entries, b = 8: 1.12 against 0.96 ms per product)
+  const bool fast16 = csr->packed == 2 && csc->packed == 2 && std::max(n, m) <= ((int64_t)1 << 26);
+  if (b <= 8 && !fast16) {
     SG_APPLY_PANEL(8)
   } else if (b <= 16) {
     SG_APPLY_PANEL(16)

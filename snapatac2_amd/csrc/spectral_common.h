@@ -71,6 +71,9 @@ namespace panel {
 // adjoint over that layout in spectral.hip).
 void product16_scaled(const snapgpu_panel_layout& L, const float* dense, float* partial, const float* scale,
                       float* out, hipStream_t st);
+// The same for 32-column rows.
+void product32_scaled(const snapgpu_panel_layout& L, const float* dense, float* partial, const float* scale,
+                      float* out, hipStream_t st);
 }  // namespace panel
 
 namespace window {
