@@ -293,7 +293,8 @@ int snapgpu_spectral_apply(const int64_t* d_indptr, const int32_t* d_idx, const 
  * the weighting of embedding.rs:314-326): dw = d<G, A(w) V>/dw, including the
  * row-norm and degree dependence on w. d_s, d_dinv, d_r32, d_w2 are the
  * outputs of snapgpu_spectral_prepare for the same d_w. The derivative with
- * respect to V is A G (A is symmetric): call snapgpu_spectral_apply on G.
+ * respect to V is A G (A is symmetric): snapgpu_spectral_apply on G, or both at
+ * once by snapgpu_spectral_vjp.
  * Workspace: snapgpu_spectral_vjp_workspace_bytes(n, m). */
 int64_t snapgpu_spectral_vjp_workspace_bytes(int64_t n, int64_t m);
 int snapgpu_spectral_vjp_w(const int64_t* d_indptr, const int32_t* d_idx, const uint32_t* d_cnt,
@@ -435,7 +436,8 @@ int snapgpu_spectral_apply_mixed(const snapgpu_window_layout* csr, const snapgpu
  * panel layout and the CSR window layout of snapgpu_spectral_apply_mixed), for
  * integer counts and b <= 8; the FP64 passes read the CSR and CSC arrays as
  * above. d_pws: snapgpu_spectral_vjp_mixed_workspace_bytes(csc n_pairs) bytes for
- * the panel product's pair sums (the mixed apply's workspace is large enough). */
+ * the panel product's pair sums (the mixed apply's workspace is large enough). The
+ * same as snapgpu_spectral_vjp without d_dV. */
 int64_t snapgpu_spectral_vjp_mixed_workspace_bytes(int64_t pairs_csc);
 int snapgpu_spectral_vjp_w_mixed(const snapgpu_window_layout* csr_windows,
                                  const snapgpu_panel_layout* csc_panels, const int64_t* d_indptr,
@@ -446,6 +448,24 @@ int snapgpu_spectral_vjp_w_mixed(const snapgpu_window_layout* csr_windows,
                                  const float* d_w2, const double* d_V, int64_t ldv, const double* d_G,
                                  int64_t ldg, int32_t b, double* d_dw, void* d_ws, int64_t ws_bytes,
                                  void* d_pws, int64_t pws_bytes, void* stream);
+
+/* Both halves of the adjoint: dw as snapgpu_spectral_vjp_w and, when d_dV is not
+ * NULL, dV = A G (n x b, row stride lddv) from the same products. The FP32
+ * products run over csc_panels and the CSR as csr_windows (integer counts, b <= 16)
+ * or csr_panels, or row-parallel when all three layouts are NULL; the FP64 passes
+ * read the CSR and CSC arrays. d_pws: with layouts,
+ * snapgpu_spectral_vjp_products_workspace_bytes(pairs of csr_panels or 0, pairs of
+ * csc_panels, b) bytes. */
+int64_t snapgpu_spectral_vjp_products_workspace_bytes(int64_t pairs_csr, int64_t pairs_csc, int32_t b);
+int snapgpu_spectral_vjp(const snapgpu_window_layout* csr_windows, const snapgpu_panel_layout* csr_panels,
+                         const snapgpu_panel_layout* csc_panels, const int64_t* d_indptr,
+                         const int32_t* d_idx, const uint32_t* d_cnt, int64_t n,
+                         const int64_t* d_colptr, const int32_t* d_rowidx, const uint32_t* d_ccnt,
+                         int64_t m, const double* d_w, const double* d_s, const double* d_dinv,
+                         const float* d_r32, const float* d_w2, const double* d_V, int64_t ldv,
+                         const double* d_G, int64_t ldg, int32_t b, double* d_dw, double* d_dV,
+                         int64_t lddv, int32_t value_type, void* d_ws, int64_t ws_bytes, void* d_pws,
+                         int64_t pws_bytes, void* stream);
 
 /* Block-tiled layout (an LDS-staged form of the same products for b <= 16,
  * slower than the panel layout at a million cells). One

@@ -835,6 +835,17 @@ __global__ void adj_rows_kernel(const double* G, int64_t ldg, const double* V, i
   t[i] = ga * u[i];
 }
 
+// dV = A G from the adjoint's own X (w^2 o Q): row i is r_i times it less dinv_i G_i,
+// rounded as the operator's product rounds it.
+__global__ void dv_kernel(const float* XQ, int BW, int b, int64_t n, const float* r, const double* dinv,
+                          const double* G, int64_t ldg, double* dV, int64_t lddv) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n * b) return;
+  const int64_t i = t / b;
+  const int c = (int)(t % b);
+  dV[i * lddv + c] = (double)(XQ[i * BW + c] * r[i]) - dinv[i] * G[i * ldg + c];
+}
+
 // pair[i] = (a[i], b[i]): two vectors gathered with one 16-byte load
 __global__ void pack_pair_kernel(const double* a, const double* b, int64_t n, double2* pair) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -925,20 +936,31 @@ static int64_t vjp_ws_bytes(int64_t n, int64_t m) {
   return 2 * al(n * kB * 4) + 2 * al(m * kB * 4) + 5 * al(n * 8) + 4 * al(m * 8) + 256;
 }
 
-// The two FP32 products of the adjoint over the mixed layout (CSC panels, CSR
-// windows) instead of the row-parallel spmm_kernel; 16-column rows only.
-struct MixedProducts {
-  const snapgpu_window_layout* csr;
+// The layouts that the adjoint's FP32 products run over instead of the
+// row-parallel spmm_kernel: the CSC as panels, the CSR as windows (16 columns) or
+// panels. 130M entries, 16 columns: 1.53 ms per product row-parallel, 0.96 over panels.
+struct Products {
+  const snapgpu_window_layout* csr_windows;
+  const snapgpu_panel_layout* csr_panels;
   const snapgpu_panel_layout* csc;
-  float* partial;  // the CSC panel product's pair sums
+  float* partial;  // the panel products' pair sums
 };
+
+template <int BW>
+static void panel_product(const snapgpu_panel_layout& L, const float* dense, float* partial, float* out,
+                          hipStream_t st) {
+  static_assert(BW == 16 || BW == 32, "panel widths of the adjoint");
+  if (BW == 16) panel::product16_scaled(L, dense, partial, nullptr, out, st);
+  else panel::product32_scaled(L, dense, partial, nullptr, out, st);
+}
 
 template <int BW, bool FV>
 static void launch_vjp(const int64_t* indptr, const int32_t* idx, const uint32_t* cnt, int64_t n,
                        const int64_t* colptr, const int32_t* rowidx, const uint32_t* ccnt, int64_t m,
                        const double* u, const double* dinv, const double* w, const float* r32,
                        const float* w2, const double* V, int64_t ldv, const double* G, int64_t ldg,
-                       int b, double* dw, void* ws, hipStream_t st, const MixedProducts* mixed = nullptr) {
+                       int b, double* dw, double* dV, int64_t lddv, void* ws, hipStream_t st,
+                       const Products* over) {
   char* q = (char*)(((uintptr_t)ws + 255) & ~(uintptr_t)255);
   auto take = [&q](int64_t bytes) {
     char* p = q;
@@ -959,44 +981,60 @@ static void launch_vjp(const int64_t* indptr, const int32_t* idx, const uint32_t
   double* phi = (double*)take(m * 8);
   double* sigma = (double*)take(m * 8);
   const unsigned gn = (unsigned)ceil_div(n, 4), gm = (unsigned)ceil_div(m, 4);
+  // out = X^T dense (features gather cells) and out = X dense
+  const auto csc_product = [&](const float* dense, float* out, int cols) {
+    if constexpr (BW >= 16) {
+      if (over) {
+        panel_product<BW>(*over->csc, dense, over->partial, out, st);
+        return;
+      }
+    }
+    spmm_kernel<BW, 0, FV><<<gm, 256, 0, st>>>(colptr, rowidx, ccnt, m, dense, nullptr, out, nullptr, 0, nullptr,
+                                               nullptr, 0, cols);
+  };
+  const auto csr_product = [&](const float* dense, float* out, int cols) {
+    if constexpr (BW >= 16) {
+      if (over && over->csr_panels) {
+        panel_product<BW>(*over->csr_panels, dense, over->partial, out, st);
+        return;
+      }
+    }
+    if constexpr (BW == 16) {
+      if (over) {
+        window::product16_scaled(*over->csr_windows, dense, nullptr, out, st);
+        return;
+      }
+    }
+    spmm_kernel<BW, 0, FV><<<gn, 256, 0, st>>>(indptr, idx, cnt, n, dense, nullptr, out, nullptr, 0, nullptr,
+                                               nullptr, 0, cols);
+  };
+  const float* XQ;  // X (w^2 o Q), rows of BW floats
   if (2 * b <= BW) {
     // V and G side by side: one CSC and one CSR pass
     scale_in_pair_kernel<BW><<<(unsigned)ceil_div(n * BW, 256), 256, 0, st>>>(V, ldv, G, ldg, n, b, r32, Vs);
-    // [P | Q] = X^T (r o [V | G])
-    if (BW == 16 && mixed)
-      panel::product16_scaled(*mixed->csc, Vs, mixed->partial, nullptr, Pm, st);
-    else
-      spmm_kernel<BW, 0, FV><<<gm, 256, 0, st>>>(colptr, rowidx, ccnt, m, Vs, nullptr, Pm, nullptr, 0,
-                                                 nullptr, nullptr, 0, 2 * b);
+    csc_product(Vs, Pm, 2 * b);  // [P | Q] = X^T (r o [V | G])
     rowdot_f32_kernel<<<(unsigned)ceil_div(m, 256), 256, 0, st>>>(Pm, Pm + b, m, BW, b, h);
     scale_rows_f32_kernel<<<(unsigned)ceil_div(m * BW, 256), 256, 0, st>>>(Pm, m, BW, w2);
-    // X (w^2 o [P | Q]) into Vs (free after the CSC pass)
-    if (BW == 16 && mixed)
-      window::product16_scaled(*mixed->csr, Pm, nullptr, Vs, st);
-    else
-      spmm_kernel<BW, 0, FV><<<gn, 256, 0, st>>>(indptr, idx, cnt, n, Pm, nullptr, Vs, nullptr, 0,
-                                                 nullptr, nullptr, 0, 2 * b);
-    adj_rows_kernel<<<(unsigned)ceil_div(n, 256), 256, 0, st>>>(G, ldg, V, ldv, Vs, Vs + b, BW, b, n, u,
+    csr_product(Pm, Vs, 2 * b);  // X (w^2 o [P | Q]) into Vs (free after the CSC pass)
+    XQ = Vs + b;
+    adj_rows_kernel<<<(unsigned)ceil_div(n, 256), 256, 0, st>>>(G, ldg, V, ldv, Vs, XQ, BW, b, n, u,
                                                                 dinv, alpha, gamma, t);
   } else {
     scale_in_kernel<BW><<<(unsigned)ceil_div(n * BW, 256), 256, 0, st>>>(V, ldv, n, b, r32, Vs);
     scale_in_kernel<BW><<<(unsigned)ceil_div(n * BW, 256), 256, 0, st>>>(G, ldg, n, b, r32, Gs);
-    // P = X^T (r o V), Q = X^T (r o G)
-    spmm_kernel<BW, 0, FV><<<gm, 256, 0, st>>>(colptr, rowidx, ccnt, m, Vs, nullptr, Pm, nullptr, 0,
-                                               nullptr, nullptr, 0, b);
-    spmm_kernel<BW, 0, FV><<<gm, 256, 0, st>>>(colptr, rowidx, ccnt, m, Gs, nullptr, Qm, nullptr, 0,
-                                               nullptr, nullptr, 0, b);
+    csc_product(Vs, Pm, b);  // P = X^T (r o V), Q = X^T (r o G)
+    csc_product(Gs, Qm, b);
     rowdot_f32_kernel<<<(unsigned)ceil_div(m, 256), 256, 0, st>>>(Pm, Qm, m, BW, b, h);
     scale_rows_f32_kernel<<<(unsigned)ceil_div(m * BW, 256), 256, 0, st>>>(Pm, m, BW, w2);
     scale_rows_f32_kernel<<<(unsigned)ceil_div(m * BW, 256), 256, 0, st>>>(Qm, m, BW, w2);
-    // X (w^2 o P) into Vs and X (w^2 o Q) into Gs (both free after the CSC pass)
-    spmm_kernel<BW, 0, FV><<<gn, 256, 0, st>>>(indptr, idx, cnt, n, Pm, nullptr, Vs, nullptr, 0,
-                                               nullptr, nullptr, 0, b);
-    spmm_kernel<BW, 0, FV><<<gn, 256, 0, st>>>(indptr, idx, cnt, n, Qm, nullptr, Gs, nullptr, 0,
-                                               nullptr, nullptr, 0, b);
-    adj_rows_kernel<<<(unsigned)ceil_div(n, 256), 256, 0, st>>>(G, ldg, V, ldv, Vs, Gs, BW, b, n, u, dinv,
+    csr_product(Pm, Vs, b);  // X (w^2 o P) into Vs and X (w^2 o Q) into Gs (both free after the CSC pass)
+    csr_product(Qm, Gs, b);
+    XQ = Gs;
+    adj_rows_kernel<<<(unsigned)ceil_div(n, 256), 256, 0, st>>>(G, ldg, V, ldv, Vs, XQ, BW, b, n, u, dinv,
                                                                 alpha, gamma, t);
   }
+  if (dV)
+    dv_kernel<<<(unsigned)ceil_div(n * b, 256), 256, 0, st>>>(XQ, BW, b, n, r32, dinv, G, ldg, dV, lddv);
   // phi = X^T (gamma o u) and e = X^T u in one pass over the CSC
   // (t, u) side by side in Gs and (w^2, phi) in Qm, both free by now
   double2* tu = reinterpret_cast<double2*>(Gs);
@@ -1326,41 +1364,89 @@ int snapgpu_spectral_apply(const int64_t* d_indptr, const int32_t* d_idx, const 
 
 int64_t snapgpu_spectral_vjp_workspace_bytes(int64_t n, int64_t m) { return vjp_ws_bytes(n, m); }
 
-int snapgpu_spectral_vjp_w(const int64_t* d_indptr, const int32_t* d_idx, const uint32_t* d_cnt, int64_t n,
-                           const int64_t* d_colptr, const int32_t* d_rowidx, const uint32_t* d_ccnt,
-                           int64_t m, const double* d_w, const double* d_s, const double* d_dinv,
-                           const float* d_r32, const float* d_w2, const double* d_V, int64_t ldv,
-                           const double* d_G, int64_t ldg, int32_t b, double* d_dw, int32_t value_type,
-                           void* d_ws, int64_t ws_bytes, void* stream) {
+int64_t snapgpu_spectral_vjp_products_workspace_bytes(int64_t pairs_csr, int64_t pairs_csc, int32_t b) {
+  return (std::max<int64_t>(std::max(pairs_csr, pairs_csc), 1) * (b <= 16 ? 16 : 32) * 4 + 255) / 256 * 256 + 256;
+}
+
+int snapgpu_spectral_vjp(const snapgpu_window_layout* csr_windows, const snapgpu_panel_layout* csr_panels,
+                         const snapgpu_panel_layout* csc_panels, const int64_t* d_indptr, const int32_t* d_idx,
+                         const uint32_t* d_cnt, int64_t n, const int64_t* d_colptr, const int32_t* d_rowidx,
+                         const uint32_t* d_ccnt, int64_t m, const double* d_w, const double* d_s,
+                         const double* d_dinv, const float* d_r32, const float* d_w2, const double* d_V,
+                         int64_t ldv, const double* d_G, int64_t ldg, int32_t b, double* d_dw, double* d_dV,
+                         int64_t lddv, int32_t value_type, void* d_ws, int64_t ws_bytes, void* d_pws,
+                         int64_t pws_bytes, void* stream) {
   clear_error();
   SG_ARG(n >= 1 && m >= 1, "bad shape");
   SG_ARG(b >= 1 && b <= kB, "block width must be in [1, 32]");
   SG_ARG(value_type == 0 || value_type == 1, "value_type must be 0 (uint32) or 1 (float32)");
-  SG_ARG(ldv >= b && ldg >= b, "leading dimension < b");
+  SG_ARG(ldv >= b && ldg >= b && (d_dV == nullptr || lddv >= b), "leading dimension < b");
   SG_ARG(d_ws != nullptr && ws_bytes >= vjp_ws_bytes(n, m), "workspace too small");
-  hipStream_t st = as_stream(stream);
   const bool fv = value_type == 1;
-#define SG_VJP(BW)                                                                                   \
-  if (fv) launch_vjp<BW, true>(d_indptr, d_idx, d_cnt, n, d_colptr, d_rowidx, d_ccnt, m, d_s, d_dinv, \
-                               d_w, d_r32, d_w2, d_V, ldv, d_G, ldg, b, d_dw, d_ws, st);            \
-  else launch_vjp<BW, false>(d_indptr, d_idx, d_cnt, n, d_colptr, d_rowidx, d_ccnt, m, d_s, d_dinv,   \
-                             d_w, d_r32, d_w2, d_V, ldv, d_G, ldg, b, d_dw, d_ws, st);
-  // width of the FP32 operand rows: V and G side by side while 2b fits 32
-  const int need = b <= 16 ? 2 * b : b;
-  if (need <= 8) {
-    SG_VJP(8)
-  } else if (need <= 16) {
-    SG_VJP(16)
+  Products over{csr_windows, csr_panels, csc_panels, nullptr};
+  if (csc_panels) {
+    SG_ARG((csr_windows != nullptr) != (csr_panels != nullptr), "give the CSR as windows or as panels");
+    SG_ARG(csc_panels->n_rows == m && csc_panels->dense_rows == n &&
+               (csr_windows ? csr_windows->n_rows == n && csr_windows->dense_rows == m
+                            : csr_panels->n_rows == n && csr_panels->dense_rows == m),
+           "layouts do not describe this matrix and its transpose");
+    SG_ARG(csc_panels->packed >= 0 && csc_panels->packed <= 2 && csc_panels->value_type == value_type &&
+               (csr_windows ? value_type == 0
+                            : csr_panels->packed >= 0 && csr_panels->packed <= 2 &&
+                                  csr_panels->value_type == value_type),
+           "layouts hold another value type");
+    SG_ARG(csr_panels || b <= 16, "block width must be in [1, 16] over windows");
+    SG_ARG(d_pws != nullptr && pws_bytes >= snapgpu_spectral_vjp_products_workspace_bytes(
+                                                csr_panels ? csr_panels->n_pairs : 0, csc_panels->n_pairs, b),
+           "panel workspace too small");
+    over.partial = reinterpret_cast<float*>(((uintptr_t)d_pws + 255) & ~(uintptr_t)255);
   } else {
-    SG_VJP(32)
+    SG_ARG(csr_windows == nullptr && csr_panels == nullptr, "a CSR layout needs the CSC panels");
+  }
+  hipStream_t st = as_stream(stream);
+  const Products* po = csc_panels ? &over : nullptr;
+#define SG_VJP(BW)                                                                                    \
+  if (fv) launch_vjp<BW, true>(d_indptr, d_idx, d_cnt, n, d_colptr, d_rowidx, d_ccnt, m, d_s, d_dinv, \
+                               d_w, d_r32, d_w2, d_V, ldv, d_G, ldg, b, d_dw, d_dV, lddv, d_ws, st, po); \
+  else launch_vjp<BW, false>(d_indptr, d_idx, d_cnt, n, d_colptr, d_rowidx, d_ccnt, m, d_s, d_dinv,   \
+                             d_w, d_r32, d_w2, d_V, ldv, d_G, ldg, b, d_dw, d_dV, lddv, d_ws, st, po);
+  if (po) {
+    // 16 columns, the products' fastest width: V and G side by side up to b = 8, one
+    // after the other up to 16
+    if (b <= 16) {
+      SG_VJP(16)
+    } else {
+      SG_VJP(32)
+    }
+  } else {
+    // width of the FP32 operand rows: V and G side by side while 2b fits 32
+    const int need = b <= 16 ? 2 * b : b;
+    if (need <= 8) {
+      SG_VJP(8)
+    } else if (need <= 16) {
+      SG_VJP(16)
+    } else {
+      SG_VJP(32)
+    }
   }
 #undef SG_VJP
   SG_LAUNCH_CHECK();
   return SNAPGPU_OK;
 }
 
+int snapgpu_spectral_vjp_w(const int64_t* d_indptr, const int32_t* d_idx, const uint32_t* d_cnt, int64_t n,
+                           const int64_t* d_colptr, const int32_t* d_rowidx, const uint32_t* d_ccnt,
+                           int64_t m, const double* d_w, const double* d_s, const double* d_dinv,
+                           const float* d_r32, const float* d_w2, const double* d_V, int64_t ldv,
+                           const double* d_G, int64_t ldg, int32_t b, double* d_dw, int32_t value_type,
+                           void* d_ws, int64_t ws_bytes, void* stream) {
+  return snapgpu_spectral_vjp(nullptr, nullptr, nullptr, d_indptr, d_idx, d_cnt, n, d_colptr, d_rowidx, d_ccnt, m,
+                              d_w, d_s, d_dinv, d_r32, d_w2, d_V, ldv, d_G, ldg, b, d_dw, nullptr, 0, value_type,
+                              d_ws, ws_bytes, nullptr, 0, stream);
+}
+
 int64_t snapgpu_spectral_vjp_mixed_workspace_bytes(int64_t pairs_csc) {
-  return (std::max<int64_t>(pairs_csc, 1) * 16 * 4 + 255) / 256 * 256 + 256;
+  return snapgpu_spectral_vjp_products_workspace_bytes(0, pairs_csc, 16);
 }
 
 int snapgpu_spectral_vjp_w_mixed(const snapgpu_window_layout* csr_windows, const snapgpu_panel_layout* csc_panels,
@@ -1372,24 +1458,10 @@ int snapgpu_spectral_vjp_w_mixed(const snapgpu_window_layout* csr_windows, const
                                  int64_t ws_bytes, void* d_pws, int64_t pws_bytes, void* stream) {
   clear_error();
   SG_ARG(csr_windows != nullptr && csc_panels != nullptr, "null layout");
-  SG_ARG(n >= 1 && m >= 1, "bad shape");
-  SG_ARG(csr_windows->n_rows == n && csr_windows->dense_rows == m && csc_panels->n_rows == m &&
-             csc_panels->dense_rows == n,
-         "layouts do not describe this matrix and its transpose");
-  SG_ARG(csc_panels->packed >= 0 && csc_panels->packed <= 2 && csc_panels->value_type == 0,
-         "the mixed layout holds integer counts");
   SG_ARG(b >= 1 && b <= 8, "block width must be in [1, 8] (V and G side by side in 16 columns)");
-  SG_ARG(ldv >= b && ldg >= b, "leading dimension < b");
-  SG_ARG(d_ws != nullptr && ws_bytes >= vjp_ws_bytes(n, m), "workspace too small");
-  SG_ARG(d_pws != nullptr && pws_bytes >= snapgpu_spectral_vjp_mixed_workspace_bytes(csc_panels->n_pairs),
-         "panel workspace too small");
-  hipStream_t st = as_stream(stream);
-  MixedProducts mp{csr_windows, csc_panels,
-                   reinterpret_cast<float*>(((uintptr_t)d_pws + 255) & ~(uintptr_t)255)};
-  launch_vjp<16, false>(d_indptr, d_idx, d_cnt, n, d_colptr, d_rowidx, d_ccnt, m, d_s, d_dinv, d_w, d_r32, d_w2,
-                        d_V, ldv, d_G, ldg, b, d_dw, d_ws, st, &mp);
-  SG_LAUNCH_CHECK();
-  return SNAPGPU_OK;
+  return snapgpu_spectral_vjp(csr_windows, nullptr, csc_panels, d_indptr, d_idx, d_cnt, n, d_colptr, d_rowidx, d_ccnt,
+                              m, d_w, d_s, d_dinv, d_r32, d_w2, d_V, ldv, d_G, ldg, b, d_dw, nullptr, 0, 0, d_ws,
+                              ws_bytes, d_pws, pws_bytes, stream);
 }
 
 int64_t snapgpu_gemm_tn_workspace_bytes(int64_t n, int32_t ka, int32_t kb) {

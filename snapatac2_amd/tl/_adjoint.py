@@ -57,9 +57,11 @@ def _function():
             op = ctx.op
             _sync_weights(op, ctx.w)
             G64 = G.detach().to(torch.float64).contiguous()
-            dV = op.matmat(G64).to(G.dtype) if ctx.needs_input_grad[0] else None
-            dw = op.vjp_w(V64, G64) if ctx.needs_input_grad[1] else None
-            return dV, dw, None
+            if ctx.needs_input_grad[1]:  # dV comes with it from the same products
+                dw, dV = op.vjp(V64, G64, want_dv=ctx.needs_input_grad[0])
+            else:
+                dw, dV = None, op.matmat(G64) if ctx.needs_input_grad[0] else None
+            return None if dV is None else dV.to(G.dtype), dw, None
 
     return NormalizedCosine
 

@@ -185,6 +185,7 @@ class SpectralOperator:
         self.n_columns = 0
         self.events = None  # optional list collecting (start, end) events per application
         self._vjp_ws = None
+        self._vjp_pws = None
 
     def _build_panel(self, ptr, idx, val, nrows: int, dense_rows: int, nnz: int):
         """Panel-major copy of one storage direction (see snapgpu_panel_build)."""
@@ -318,6 +319,11 @@ class SpectralOperator:
 
     def vjp_w(self, V, G):
         """dw = d<G, A(w) V>/dw (FP64 device vector of length m) for FP64 n x b blocks."""
+        return self.vjp(V, G, want_dv=False)[0]
+
+    def vjp(self, V, G, want_dv: bool = True):
+        """(dw, dV): d<G, A(w) V>/dw and, if wanted, d<G, A(w) V>/dV = A(w) G from the
+        same sparse products (None otherwise)."""
         torch = self.torch
         L = _lib.lib()
         X = self.X
@@ -328,35 +334,37 @@ class SpectralOperator:
         if self._vjp_ws is None:
             self._vjp_ws_b = int(L.snapgpu_spectral_vjp_workspace_bytes(self.n, self.m))
             self._vjp_ws = torch.empty(self._vjp_ws_b, dtype=torch.uint8, device=self.w.device)
+        csr_w = csr_p = csc_p = None
+        pws, pws_b = None, 0
+        if self.layout == "mixed":
+            csr_w, csc_p = C.byref(self.window_csr), C.byref(self.panel_csc)
+            pws, pws_b = self._pws, self._pws_b
+        elif self.layout == "panel":
+            csr_p, csc_p = C.byref(self.panel_csr), C.byref(self.panel_csc)
+            need = int(L.snapgpu_spectral_vjp_products_workspace_bytes(self.panel_csr.n_pairs, self.panel_csc.n_pairs,
+                                                                       min(V.shape[1], 32)))
+            if self._vjp_pws is None or self._vjp_pws.numel() < need:
+                self._vjp_pws = torch.empty(need, dtype=torch.uint8, device=self.w.device)
+            pws, pws_b = self._vjp_pws, self._vjp_pws.numel()
         dw = torch.zeros(self.m, dtype=torch.float64, device=self.w.device)
-        mixed = self.layout == "mixed"
-        step = 8 if mixed else 32  # the mixed products take V and G side by side in 16 columns
+        dV = torch.empty(G.shape, dtype=torch.float64, device=self.w.device) if want_dv else None
+        step = 16 if csr_w is not None else 32  # columns per call
         part = torch.empty_like(dw) if V.shape[1] > step else dw
         for c0 in range(0, V.shape[1], step):
             b = min(step, V.shape[1] - c0)
             Vc, Gc = V[:, c0:c0 + b], G[:, c0:c0 + b]
-            if mixed:
-                _lib.check(L.snapgpu_spectral_vjp_w_mixed(
-                    C.byref(self.window_csr), C.byref(self.panel_csc),
-                    X.indptr.data_ptr(), X.indices.data_ptr(), X.data.data_ptr(), self.n,
-                    self.colptr.data_ptr(), self.rowidx.data_ptr(), self.cval.data_ptr(), self.m,
-                    self.w.data_ptr(), self.s.data_ptr(), self.dinv.data_ptr(), self.r32.data_ptr(),
-                    self.w2.data_ptr(), Vc.data_ptr(), Vc.stride(0), Gc.data_ptr(), Gc.stride(0), b,
-                    part.data_ptr(), self._vjp_ws.data_ptr(), self._vjp_ws_b, self._pws.data_ptr(),
-                    self._pws_b, _lib.stream_ptr()))
-                if part is not dw:
-                    dw += part
-                continue
-            _lib.check(L.snapgpu_spectral_vjp_w(
+            dVc = dV[:, c0:c0 + b] if want_dv else None
+            _lib.check(L.snapgpu_spectral_vjp(
+                csr_w, csr_p, csc_p,
                 X.indptr.data_ptr(), X.indices.data_ptr(), X.data.data_ptr(), self.n,
                 self.colptr.data_ptr(), self.rowidx.data_ptr(), self.cval.data_ptr(), self.m,
                 self.w.data_ptr(), self.s.data_ptr(), self.dinv.data_ptr(), self.r32.data_ptr(),
                 self.w2.data_ptr(), Vc.data_ptr(), Vc.stride(0), Gc.data_ptr(), Gc.stride(0), b,
-                part.data_ptr(), self.value_type, self._vjp_ws.data_ptr(), self._vjp_ws_b,
-                _lib.stream_ptr()))
+                part.data_ptr(), _lib.ptr(dVc), dVc.stride(0) if want_dv else 0, self.value_type,
+                self._vjp_ws.data_ptr(), self._vjp_ws_b, _lib.ptr(pws), pws_b, _lib.stream_ptr()))
             if part is not dw:
                 dw += part
-        return dw
+        return dw, dV
 
     def apply(self, V, Y, b: int | None = None) -> None:
         """Y[:, :b] = A V[:, :b]; V, Y row-major FP64 device tensors (any row stride)."""
