@@ -710,6 +710,14 @@ int snapgpu_peak_pairs(const snapgpu_peak_index* index, const int64_t* d_cell_pt
 int snapgpu_peak_csr(const void* d_ws, int64_t ws_bytes, int64_t total, int64_t nnz, int64_t n_cells,
                      int64_t* d_indptr, int32_t* d_idx, uint32_t* d_val, void* stream);
 
+/* What spectral() returns of its eigenvectors (_embedding.py:284-288): columns
+ * d_cols[kc] of d_U (n rows, row stride ldu), each with the sign that makes its
+ * entry of largest magnitude (the first of equal ones) positive, times d_scale[kc]
+ * if not NULL, as n x kc rows in d_out. */
+int64_t snapgpu_embed_workspace_bytes(int64_t n, int32_t kc);
+int snapgpu_embed_finish(const double* d_U, int64_t ldu, int64_t n, const int32_t* d_cols, int32_t kc,
+                         const double* d_scale, double* d_out, void* d_ws, int64_t ws_bytes, void* stream);
+
 /* Gene level of the gene matrix (create_gene_matrix with id_type "gene",
  * feature_count/matrix.rs:173-273; GeneCount::get_values, counter.rs:270-283):
  * each row's entries grouped by d_group[column] (the gene of the region's

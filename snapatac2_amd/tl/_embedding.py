@@ -12,7 +12,7 @@ from typing import Literal
 import numpy as np
 
 from .. import _lib
-from ._lanczos import _fix_signs, eigsh_lm
+from ._lanczos import eigsh_lm
 from ._operator import SpectralOperator, _to_device_csr, select_columns
 
 
@@ -34,11 +34,30 @@ def _selected_columns(features, n_vars: int):
     return f[perm], perm
 
 
-def spectral_embedding(adata, features, n_components: int, random_state: int = 0,
-                       feature_weights=None, return_stats: bool = False, device_output: bool = False):
-    """(evals, evecs) of the matrix-free normalized cosine operator, like the
-    reference's internal.spectral_embedding: eigenpairs of largest magnitude,
-    sorted by descending eigenvalue."""
+def _finished(U, cols, scale=None) -> np.ndarray:
+    """Columns `cols` of the device matrix U, signed (largest-magnitude entry positive)
+    and scaled on the device (snapgpu_embed_finish), as a host array."""
+    torch = _lib.require_gpu()
+    L = _lib.lib()
+    n, kc = U.shape[0], len(cols)
+    if U.stride(1) != 1:
+        U = U.contiguous()
+    d_cols = torch.from_numpy(np.asarray(cols, dtype=np.int32)).to(U.device)
+    d_scale = None if scale is None else torch.from_numpy(np.asarray(scale, dtype=np.float64)).to(U.device)
+    out = torch.empty((n, kc), dtype=torch.float64, device=U.device)
+    ws_b = int(L.snapgpu_embed_workspace_bytes(n, kc))
+    ws = torch.empty(ws_b, dtype=torch.uint8, device=U.device)
+    _lib.check(L.snapgpu_embed_finish(U.data_ptr(), U.stride(0), n, d_cols.data_ptr(), kc, _lib.ptr(d_scale),
+                                      out.data_ptr(), ws.data_ptr(), ws_b, _lib.stream_ptr()))
+    # page-locked (the returned array keeps it alive): one DMA
+    host = torch.empty((n, kc), dtype=torch.float64, pin_memory=True)
+    host.copy_(out, non_blocking=True)
+    torch.cuda.current_stream().synchronize()
+    return host.numpy()
+
+
+def _eigenpairs(adata, features, n_components: int, random_state: int, feature_weights):
+    """(evals descending, U, the columns of U in that order, solver statistics)."""
     torch = _lib.require_gpu()
     X = _to_device_csr(adata.X, torch)
     cols, perm = _selected_columns(features, X.shape[1])
@@ -51,12 +70,20 @@ def spectral_embedding(adata, features, n_components: int, random_state: int = 0
     op = SpectralOperator(Xs, w)
     evals, U, stats = eigsh_lm(op, n_components, seed=random_state)
     ix = np.argsort(evals, kind="stable")[::-1]
-    evals = evals[ix]
-    U = U[:, torch.from_numpy(ix.copy()).to(U.device)]
+    return evals[ix], U, ix, stats
+
+
+def spectral_embedding(adata, features, n_components: int, random_state: int = 0,
+                       feature_weights=None, return_stats: bool = False, device_output: bool = False):
+    """(evals, evecs) of the matrix-free normalized cosine operator, like the
+    reference's internal.spectral_embedding: eigenpairs of largest magnitude,
+    sorted by descending eigenvalue."""
+    torch = _lib.require_gpu()
+    evals, U, ix, stats = _eigenpairs(adata, features, n_components, random_state, feature_weights)
     if device_output:
-        evecs = U
+        evecs = U[:, torch.from_numpy(ix.copy()).to(U.device)]
     else:
-        evecs = _fix_signs(U.cpu().numpy())
+        evecs = _finished(U, ix)
     if return_stats:
         return evals, evecs, stats
     return evals, evecs
@@ -115,14 +142,16 @@ def spectral(
         # the reference's Nystrom call takes no feature weights: always IDF
         v, u = spectral_embedding_nystrom(select_columns(X, cols), n_comps, sample_size,
                                           sample_method != "random", chunk_size)
-        evals, evecs = orthogonalize(v, u)
-        evecs = _fix_signs(evecs.cpu().numpy())
+        evals, U = orthogonalize(v, u)
+        order = np.arange(evals.shape[0])
     else:
-        evals, evecs = spectral_embedding(adata, features, n_comps, random_state, feature_weights)
+        evals, U, order, _ = _eigenpairs(adata, features, n_comps, random_state, feature_weights)
     if weighted_by_sd:
         idx = [i for i in range(evals.shape[0]) if evals[i] > 0]
         evals = evals[idx]
-        evecs = evecs[:, idx] * np.sqrt(evals)
+        evecs = _finished(U, order[idx], np.sqrt(evals))
+    else:
+        evecs = _finished(U, order)
     if inplace:
         adata.uns["spectral_eigenvalue"] = evals
         adata.obsm["X_spectral"] = evecs

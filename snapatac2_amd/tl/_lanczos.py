@@ -78,14 +78,6 @@ def _lm_order(theta: np.ndarray, k: int) -> np.ndarray:
     return np.lexsort((-theta, -np.abs(theta)))[:k]
 
 
-def _fix_signs(U: np.ndarray) -> np.ndarray:
-    """Deterministic sign convention: the largest-magnitude entry of each vector is positive."""
-    idx = np.argmax(np.abs(U), axis=0)
-    sg = np.sign(U[idx, np.arange(U.shape[1])])
-    sg[sg == 0] = 1.0
-    return U * sg
-
-
 def dense_eigsh(op, k: int):
     """All-pairs path for small n: A assembled column-block by column-block on the device."""
     torch = op.torch
