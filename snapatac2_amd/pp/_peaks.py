@@ -45,37 +45,78 @@ def parse_regions(peaks) -> tuple[list[str], list[tuple[str, int, int]]]:
     return names, regs
 
 
+class RegionArrays:
+    """Distinct regions as arrays: chromosome id among `chroms` (-1: none of them),
+    start and end; column j = region j."""
+
+    def __init__(self, chrom, start, end):
+        self.chrom, self.start, self.end = chrom, start, end
+
+    def __len__(self) -> int:
+        return len(self.start)
+
+    @classmethod
+    def of(cls, regs, chroms) -> "RegionArrays":
+        cid = {c: i for i, c in enumerate(chroms)}
+        n = len(regs)
+        return cls(np.fromiter((cid.get(r[0], -1) for r in regs), dtype=np.int32, count=n),
+                   np.fromiter((r[1] for r in regs), dtype=np.int64, count=n),
+                   np.fromiter((r[2] for r in regs), dtype=np.int64, count=n))
+
+
+def parse_region_arrays(peaks, chroms) -> tuple[list[str], RegionArrays]:
+    """parse_regions, as arrays: in native code when every item is plain
+    "chrom:start-end", else through parse_regions (blanks, signs, other digits,
+    errors)."""
+    L = _lib.lib()
+    items = [str(p) for p in peaks]
+    n = len(items)
+    text = "\n".join(items).encode("utf-8", "surrogatepass")
+    encoded = [c.encode("utf-8", "surrogatepass") for c in chroms]
+    chrom = np.empty(n, dtype=np.int32)
+    start, end, first = (np.empty(n, dtype=np.int64) for _ in range(3))
+    names = (C.c_char_p * max(len(chroms), 1))(*encoded)
+    kept, plain = C.c_int64(0), C.c_int32(0)
+    _lib.check(L.snapgpu_region_parse(text, len(text), n, names, len(chroms), chrom.ctypes.data, start.ctypes.data,
+                                      end.ctypes.data, first.ctypes.data, C.byref(kept), C.byref(plain)))
+    if not plain.value or any(b"\0" in c for c in encoded):
+        found, regs = parse_regions(items)
+        return found, RegionArrays.of(regs, chroms)
+    k = kept.value
+    if k < n:
+        items = [items[i] for i in first[:k].tolist()]
+    return items, RegionArrays(chrom[:k], start[:k], end[:k])
+
+
+def region_index(r: RegionArrays, n_chrom: int):
+    """(starts, ends, running maxima of the ends, region, chromosome offsets): the
+    regions of each chromosome by start and index (snapgpu_peak_index)."""
+    n = len(r)
+    size = max(n, 1)
+    starts, ends, pmax = (np.zeros(size, dtype=np.uint64) for _ in range(3))
+    index = np.zeros(size, dtype=np.uint32)
+    off = np.zeros(n_chrom + 1, dtype=np.int64)
+    chrom, start, end = (np.ascontiguousarray(a, dtype=t) for a, t in
+                         ((r.chrom, np.int32), (r.start, np.int64), (r.end, np.int64)))
+    _lib.check(_lib.lib().snapgpu_region_index(
+        chrom.ctypes.data, start.ctypes.data, end.ctypes.data, n, n_chrom, starts.ctypes.data, ends.ctypes.data,
+        pmax.ctypes.data, index.ctypes.data, off.ctypes.data))
+    return starts, ends, pmax, index, off
+
+
 class PeakIndex:
-    """The region index of snapgpu_peak_index on the device."""
+    """The region index of snapgpu_peak_index on the device, of RegionArrays or of
+    (chrom, start, end) tuples."""
 
     def __init__(self, regs, chrom_sizes: dict[str, int], torch):
         dev = torch.device("cuda")
         chroms = list(chrom_sizes)
-        cid = {c: i for i, c in enumerate(chroms)}
-        rc = np.fromiter((cid.get(r[0], -1) for r in regs), dtype=np.int64, count=len(regs))
-        rs = np.fromiter((r[1] for r in regs), dtype=np.int64, count=len(regs))
-        re_ = np.fromiter((r[2] for r in regs), dtype=np.int64, count=len(regs))
-        ri = np.arange(len(regs), dtype=np.int64)
-        on = rc >= 0
-        rc, rs, re_, ri = rc[on], rs[on], re_[on], ri[on]
-        order = np.lexsort((ri, rs, rc))
-        arr = np.stack([rc[order], rs[order], re_[order], ri[order]], axis=1).reshape(-1, 4)
-        starts = arr[:, 1].astype(np.uint64)
-        ends = arr[:, 2].astype(np.uint64)
-        pmax = np.zeros_like(ends)
-        off = np.searchsorted(arr[:, 0], np.arange(len(chroms) + 1), side="left").astype(np.int64)
-        for c in range(len(chroms)):
-            a, b = off[c], off[c + 1]
-            if b > a:
-                pmax[a:b] = np.maximum.accumulate(ends[a:b])
+        r = regs if isinstance(regs, RegionArrays) else RegionArrays.of(regs, chroms)
+        starts, ends, pmax, index, off = region_index(r, len(chroms))
         base = np.concatenate([[0], np.cumsum([int(chrom_sizes[c]) for c in chroms])]).astype(np.uint64)
         t = lambda a: torch.from_numpy(np.ascontiguousarray(a).view(np.int64 if a.dtype.itemsize == 8 else np.int32)).to(dev)
-        self._keep = [t(starts if starts.size else np.zeros(1, np.uint64)),
-                      t(ends if ends.size else np.zeros(1, np.uint64)),
-                      t(pmax if pmax.size else np.zeros(1, np.uint64)),
-                      t(arr[:, 3].astype(np.uint32) if arr.size else np.zeros(1, np.uint32)),
-                      t(off), t(base)]
-        self.c = _lib.PeakIndex(*[x.data_ptr() for x in self._keep], len(chroms), len(regs))
+        self._keep = [t(a) for a in (starts, ends, pmax, index, off, base)]
+        self.c = _lib.PeakIndex(*[x.data_ptr() for x in self._keep], len(chroms), len(r))
 
 
 def make_peak_counts(frags, chrom_sizes: dict[str, int], peaks, counting_strategy: str = "paired-insertion",
@@ -84,14 +125,14 @@ def make_peak_counts(frags, chrom_sizes: dict[str, int], peaks, counting_strateg
     if counting_strategy not in _STRATEGY:
         raise RuntimeError("Counting strategy must be one of 'insertion', 'fragment', or "
                            "'paired-insertion'")  # counter.rs:25-36
-    names, regs = parse_regions(peaks)
+    names, regs = parse_region_arrays(peaks, list(chrom_sizes))
     return region_counts(frags, chrom_sizes, regs, counting_strategy, min_frag_size, max_frag_size), names
 
 
 def region_counts(frags, chrom_sizes: dict[str, int], regs, counting_strategy: str = "paired-insertion",
                   min_frag_size: int | None = None, max_frag_size: int | None = None) -> DeviceCSR:
-    """DeviceCSR cells x len(regs) with uint32 counts; regs = distinct
-    (chrom, start, end) tuples, column j = regs[j]."""
+    """DeviceCSR cells x len(regs) with uint32 counts; regs = distinct regions as
+    RegionArrays or (chrom, start, end) tuples, column j = regs[j]."""
     torch = _lib.require_gpu()
     L = _lib.lib()
     st = _lib.stream_ptr()
@@ -107,7 +148,7 @@ def region_counts(frags, chrom_sizes: dict[str, int], regs, counting_strategy: s
     lo = 0 if min_frag_size is None else int(min_frag_size)
     hi = 0xFFFFFFFF if max_frag_size is None else int(min(max_frag_size, 0xFFFFFFFF))
     indptr = torch.zeros(n_cells + 1, dtype=torch.int64, device=dev)
-    if n_frag == 0 or n_cells == 0 or not regs:
+    if n_frag == 0 or n_cells == 0 or len(regs) == 0:
         return DeviceCSR(indptr, torch.empty(0, dtype=torch.int32, device=dev),
                          torch.empty(0, dtype=torch.int32, device=dev), (n_cells, len(regs)))
     hits = torch.empty(n_frag, dtype=torch.int64, device=dev)
