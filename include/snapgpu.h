@@ -710,6 +710,10 @@ int snapgpu_peak_pairs(const snapgpu_peak_index* index, const int64_t* d_cell_pt
 int snapgpu_peak_csr(const void* d_ws, int64_t ws_bytes, int64_t total, int64_t nnz, int64_t n_cells,
                      int64_t* d_indptr, int32_t* d_idx, uint32_t* d_val, void* stream);
 
+/* Column sums as select_features takes them (_basic.py:1053-1058): d_out[j] = d_sums[j]
+ * as a double, *d_zeros = how many of the m are zero (or below). */
+int snapgpu_col_sums_f64(const int64_t* d_sums, int64_t m, double* d_out, uint64_t* d_zeros, void* stream);
+
 /* What spectral() returns of its eigenvectors (_embedding.py:284-288): columns
  * d_cols[kc] of d_U (n rows, row stride ldu), each with the sign that makes its
  * entry of largest magnitude (the first of equal ones) positive, times d_scale[kc]

@@ -195,6 +195,26 @@ static int col_window_sums(const int64_t* d_indptr, int64_t n, const IdxT* d_idx
   return SNAPGPU_OK;
 }
 
+// out[j] = sums[j] as a double; *zeros += the sums that are not positive
+__global__ void __launch_bounds__(256) sums_f64_kernel(const int64_t* __restrict__ sums, int64_t m,
+                                                       double* __restrict__ out, unsigned long long* __restrict__ zeros) {
+  __shared__ unsigned int part[4];
+  unsigned int z = 0;
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < m; j += stride) {
+    const int64_t v = sums[j];
+    out[j] = (double)v;
+    z += v <= 0;
+  }
+  for (int o = 32; o > 0; o >>= 1) z += (unsigned int)__shfl_xor((int)z, o, 64);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = z;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    z = part[0] + part[1] + part[2] + part[3];
+    if (z) atomicAdd(zeros, (unsigned long long)z);
+  }
+}
+
 int col_counts_sorted(const int64_t* d_indptr, int64_t n, const int32_t* d_idx, int64_t nnz, int64_t m,
                       unsigned long long* d_out, int32_t* d_status, hipStream_t st, bool* sorted) {
   return col_window_sums<int32_t, true>(d_indptr, n, d_idx, nullptr, nnz, m, d_out, d_status, st, sorted);
@@ -221,6 +241,18 @@ int snapgpu_csr_col_sum_u32(const void* d_indices, int32_t index_bits, const uin
   else
     col_sum_kernel<int64_t><<<(unsigned)blocks, 256, 0, as_stream(stream)>>>(
         static_cast<const int64_t*>(d_indices), d_values, nnz, out);
+  SG_LAUNCH_CHECK();
+  return SNAPGPU_OK;
+}
+
+int snapgpu_col_sums_f64(const int64_t* d_sums, int64_t m, double* d_out, uint64_t* d_zeros, void* stream) {
+  clear_error();
+  SG_ARG(m >= 0 && d_zeros != nullptr && (m == 0 || (d_sums && d_out)), "bad arguments");
+  hipStream_t st = as_stream(stream);
+  SG_HIP(hipMemsetAsync(d_zeros, 0, 8, st));
+  if (m == 0) return SNAPGPU_OK;
+  sums_f64_kernel<<<(unsigned)std::min<int64_t>(ceil_div(m, 256), 2048), 256, 0, st>>>(
+      d_sums, m, d_out, reinterpret_cast<unsigned long long*>(d_zeros));
   SG_LAUNCH_CHECK();
   return SNAPGPU_OK;
 }

@@ -338,6 +338,14 @@ def _set_x(adata, X, var_names) -> None:
 
 def _column_sums(X) -> np.ndarray:
     """Column sums of the count matrix as float64 (exact: integer sums)."""
+    return _counted_column_sums(X)[0]
+
+
+def _counted_column_sums(X) -> tuple[np.ndarray, int]:
+    """_column_sums and how many of them are zero. The conversion and the count run
+    on the device, and the sums come to the host in page-locked memory (the returned
+    array keeps it alive). select_features on 6.06M columns: 65.5 ms with both in
+    numpy, 32.0 ms so, nearly all of it numpy's argsort."""
     torch = _lib.require_gpu()
     L = _lib.lib()
     if not isinstance(X, DeviceCSR):
@@ -355,20 +363,28 @@ def _column_sums(X) -> np.ndarray:
     _lib.check(L.snapgpu_csr_col_sum_rows_u32(X.indptr.data_ptr(), X.shape[0], X.indices.data_ptr(), bits,
                                               X.data.data_ptr(), X.shape[1], out.data_ptr(),
                                               ws.data_ptr(), _lib.stream_ptr()))
-    return out.cpu().numpy().astype(np.float64)
+    m = X.shape[1]
+    sums = torch.empty(m, dtype=torch.float64, device=X.device)
+    zeros = torch.empty(1, dtype=torch.int64, device=X.device)
+    _lib.check(L.snapgpu_col_sums_f64(out.data_ptr(), m, sums.data_ptr(), zeros.data_ptr(), _lib.stream_ptr()))
+    host = torch.empty(m, dtype=torch.float64, pin_memory=True)
+    host.copy_(sums, non_blocking=True)
+    return host.numpy(), int(zeros.item())  # item() waits for both copies
 
 
 def _find_most_accessible_features(feature_count, filter_lower_quantile, filter_upper_quantile,
-                                   total_features) -> np.ndarray:
+                                   total_features, zeros: int | None = None) -> np.ndarray:
     """Same steps as _basic.py:952-967 (numpy's default argsort, so equal counts
-    are ordered exactly as the reference orders them on the same host)."""
+    are ordered exactly as the reference orders them on the same host). zeros: how
+    many counts are not positive, if known."""
     idx = np.argsort(feature_count)
     # first position with a positive count, as the reference's loop finds it (the
     # last position when none is positive; with no features `i` stays unbound there
     # and here alike)
     if idx.size:
-        pos = np.asarray(feature_count)[idx] > 0
-        i = int(np.argmax(pos)) if pos.any() else idx.size - 1
+        if zeros is None:
+            zeros = int(np.count_nonzero(np.asarray(feature_count) <= 0))
+        i = min(zeros, idx.size - 1)
     idx = idx[i:]
     n = idx.size
     n_lower = int(filter_lower_quantile * n)
@@ -404,11 +420,11 @@ def select_features(
         return None if inplace else res
     if max_iter > 1:
         raise NotImplementedError("iterative feature selection (max_iter > 1) is not supported")
-    count = _column_sums(adata.X)
+    count, zeros = _counted_column_sums(adata.X)
     if inplace:
         adata.var["count"] = count
     selected = _find_most_accessible_features(count, filter_lower_quantile,
-                                              filter_upper_quantile, n_features)
+                                              filter_upper_quantile, n_features, zeros)
     if blacklist is not None:
         black = intersect_bed(adata.var_names, str(blacklist))
         selected = selected[np.logical_not(black[selected])]
