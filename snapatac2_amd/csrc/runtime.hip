@@ -36,37 +36,65 @@ __global__ void __launch_bounds__(kScanThreads) scan_reduce_kernel(const int64_t
   __shared__ int64_t lds[kScanThreads / 64];
   const int64_t base = (int64_t)blockIdx.x * kScanTile;
   int64_t s = 0;
+  if (base + kScanTile <= n) {  // whole tiles: all loads in flight
 #pragma unroll
-  for (int i = 0; i < kScanItems; ++i) {
-    int64_t idx = base + (int64_t)i * kScanThreads + threadIdx.x;
-    if (idx < n) s += data[idx];
+    for (int i = 0; i < kScanItems; ++i) s += data[base + i * kScanThreads + threadIdx.x];
+  } else {
+    for (int i = 0; i < kScanItems; ++i) {
+      const int64_t idx = base + (int64_t)i * kScanThreads + threadIdx.x;
+      if (idx < n) s += data[idx];
+    }
   }
   int64_t total;
   block_excl_scan(s, lds, &total);
   if (threadIdx.x == 0) block_sums[blockIdx.x] = total;
 }
 
-// Each thread owns kScanItems consecutive elements.
+// Each thread sums kScanItems consecutive elements; they reach it through LDS, so
+// that the loads and stores of a wave are consecutive too (a lane that reads its own
+// 128 bytes touches 64 lines per load and writes each of them 16 times over:
+// 490 us for 55 million elements, both passes together, 270 us so, which is the
+// memory's rate). Element e lies at e + e / kScanItems: the lanes' runs start
+// in different banks.
 __global__ void __launch_bounds__(kScanThreads) scan_apply_kernel(int64_t* data, int64_t n,
                                                                   const int64_t* block_offsets) {
   __shared__ int64_t lds[kScanThreads / 64];
-  const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
-  int64_t v[kScanItems];
+  __shared__ int64_t tile[kScanTile + kScanTile / kScanItems];
+  const int64_t base = (int64_t)blockIdx.x * kScanTile;
+  const bool whole = base + kScanTile <= n;
+  if (whole) {
+    int64_t v[kScanItems];
+#pragma unroll
+    for (int i = 0; i < kScanItems; ++i) v[i] = data[base + i * kScanThreads + threadIdx.x];
+#pragma unroll
+    for (int i = 0; i < kScanItems; ++i) {
+      const int e = i * kScanThreads + threadIdx.x;
+      tile[e + e / kScanItems] = v[i];
+    }
+  } else {
+    for (int i = 0; i < kScanItems; ++i) {
+      const int e = i * kScanThreads + threadIdx.x;
+      tile[e + e / kScanItems] = base + e < n ? data[base + e] : 0;
+    }
+  }
+  __syncthreads();
+  int64_t* own = tile + threadIdx.x * (kScanItems + 1);
   int64_t s = 0;
 #pragma unroll
   for (int i = 0; i < kScanItems; ++i) {
-    int64_t idx = base + i;
-    v[i] = idx < n ? data[idx] : 0;
-    s += v[i];
+    s += own[i];
+    own[i] = s;
   }
   int64_t total;
   int64_t off = block_excl_scan(s, lds, &total);
   if (block_offsets != nullptr && blockIdx.x > 0) off += block_offsets[blockIdx.x - 1];
 #pragma unroll
+  for (int i = 0; i < kScanItems; ++i) own[i] += off;
+  __syncthreads();
+#pragma unroll
   for (int i = 0; i < kScanItems; ++i) {
-    off += v[i];
-    int64_t idx = base + i;
-    if (idx < n) data[idx] = off;
+    const int e = i * kScanThreads + threadIdx.x;
+    if (whole || base + e < n) data[base + e] = tile[e + e / kScanItems];
   }
 }
 
