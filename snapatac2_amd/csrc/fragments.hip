@@ -12,8 +12,9 @@
 //
 // Steps (all on one stream; the host reads three scalars back in between):
 //   1. newline count per 64 KiB block, scan, newline positions -> line starts;
-//   2. one lane per line parses its fields (tab separated), looks the
-//      chromosome up in a hashed name table and writes per-line records;
+//   2. one lane per line parses its fields (tab separated; eight characters at
+//      a time where the line is an ordinary one), looks the chromosome up in a
+//      hashed name table and writes per-line records;
 //   3. the records with end > start are compacted;
 //   4. stable radix sorts put them in (barcode group, position, value) order:
 //      by (position, value) first, then by the run index of the barcode in the
@@ -27,6 +28,7 @@
 #include <hipcub/hipcub.hpp>
 
 #include <cstring>
+#include <type_traits>
 
 #include "common.h"
 
@@ -37,9 +39,6 @@ constexpr int kThreads = 256;
 constexpr int kRounds = 16;                                     // 16-byte words per thread
 constexpr int64_t kByteBlock = (int64_t)kThreads * kRounds * 16;  // 64 KiB of text per block
 constexpr int64_t kLineBlock = (int64_t)kThreads * kRounds;       // 4096 records per block
-
-constexpr uint64_t kFnvOffset = 1469598103934665603ull;
-constexpr uint64_t kFnvPrime = 1099511628211ull;
 
 // per-line flags
 constexpr uint8_t F_KEEP = 1;     // a record with end != start (import.rs:66)
@@ -99,7 +98,18 @@ struct Counters {
   unsigned int max_size;        // largest end - start (low 32 bits) over kept records
 };
 
-__host__ __device__ inline uint64_t fnv_step(uint64_t h, uint32_t c) { return (h ^ c) * kFnvPrime; }
+// Hash of a name, eight bytes at a time (little endian, zeros past the end): a
+// multiply and a shift per word on top of the length, and one more at the end.
+__host__ __device__ inline uint64_t hash_start(uint32_t len) { return 0x2545F4914F6CDD1Dull + len; }
+__host__ __device__ inline uint64_t hash_step(uint64_t h, uint64_t w) {
+  h = (h ^ w) * 0x9E3779B97F4A7C15ull;
+  return h ^ (h >> 32);
+}
+__host__ __device__ inline uint64_t hash_end(uint64_t h) {
+  h *= 0xD6E8FEB86659FD93ull;
+  return h ^ (h >> 32);
+}
+constexpr int64_t kNamePad = 8;  // readable bytes after a table's names
 
 __device__ __forceinline__ uint8_t load_byte(const uint8_t* t, int64_t p) { return t[p]; }
 
@@ -111,13 +121,53 @@ __device__ __forceinline__ uint64_t load_word(const uint8_t* t, int64_t a, int64
   return w;
 }
 
-__device__ bool bytes_equal(const uint8_t* a, const uint8_t* b, uint32_t len) {
-  for (uint32_t k = 0; k < len; ++k)
-    if (a[k] != b[k]) return false;
-  return true;
+// 8 bytes at any address (all readable).
+struct __attribute__((packed)) Bytes8 {
+  uint64_t v;
+};
+__device__ __forceinline__ uint64_t load8(const uint8_t* p) { return reinterpret_cast<const Bytes8*>(p)->v; }
+
+// The first n (1 to 8) bytes of a word.
+__device__ __forceinline__ uint64_t first_bytes(uint64_t w, uint32_t n) { return w & (~0ull >> (64 - 8 * n)); }
+
+// 8 bytes at any offset p; bytes at or past n read as 0.
+__device__ __forceinline__ uint64_t load_u8x8(const uint8_t* t, int64_t p, int64_t n) {
+  if (p + 8 <= n) return load8(t + p);
+  uint64_t w = 0;
+  for (int k = 0; k < 8 && p + k < n; ++k) w |= (uint64_t)t[p + k] << (8 * k);
+  return w;
 }
 
-__device__ int table_find(const uint8_t* tab, uint64_t h, const uint8_t* s, uint32_t len) {
+// The text where it lies, and the part of it that a block holds in LDS (from byte
+// `first`, a multiple of 16): eight bytes at any offset.
+struct FarText {
+  const uint8_t* t;
+  int64_t n;
+  __device__ __forceinline__ uint64_t at(int64_t off) const { return load_u8x8(t, off, n); }
+};
+struct NearText {
+  const uint32_t* w;
+  int64_t first;
+  __device__ __forceinline__ uint64_t at(int64_t off) const {
+    const uint32_t r = (uint32_t)(off - first), k = r >> 2;
+    const uint32_t a = w[k], b = w[k + 1], c = w[k + 2];
+    return ((uint64_t)__builtin_amdgcn_alignbyte(c, b, r & 3) << 32) | __builtin_amdgcn_alignbyte(b, a, r & 3);
+  }
+};
+
+template <typename Text>
+__device__ __forceinline__ uint64_t hash_text(const Text& t, int64_t off, uint32_t len) {
+  uint64_t h = hash_start(len);
+  for (uint32_t k = 0; k < len; k += 8) {
+    const uint64_t w = t.at(off + k);
+    h = hash_step(h, len - k < 8 ? first_bytes(w, len - k) : w);
+  }
+  return hash_end(h);
+}
+
+// Index of the name at offset off of the text in a table, or -1.
+template <typename Text>
+__device__ int table_find(const uint8_t* tab, uint64_t h, const Text& t, int64_t off, uint32_t len) {
   const TableHeader* H = reinterpret_cast<const TableHeader*>(tab);
   const uint32_t cap = H->cap, n = H->n;
   const TableSlot* S = reinterpret_cast<const TableSlot*>(tab + sizeof(TableHeader));
@@ -129,7 +179,12 @@ __device__ int table_find(const uint8_t* tab, uint64_t h, const uint8_t* s, uint
     if (sl.idx < 0) return -1;
     if (sl.hash == h) {
       const TableEntry e = E[sl.idx];
-      if (e.name_len == len && bytes_equal(names + e.name_off, s, len)) return sl.idx;
+      bool same = e.name_len == len;
+      for (uint32_t k = 0; same && k < len; k += 8) {
+        const uint64_t x = load8(names + e.name_off + k) ^ t.at(off + k);
+        same = (len - k < 8 ? first_bytes(x, len - k) : x) == 0;
+      }
+      if (same) return sl.idx;
     }
   }
   return -1;
@@ -252,7 +307,7 @@ struct ParseOut {
   uint32_t* cnt;
   uint8_t* flags;
   uint64_t* bc;   // barcode offset << 8 | length
-  uint64_t* bch;  // FNV-1a hash of the barcode
+  uint64_t* bch;  // hash of the barcode
 };
 
 __device__ __forceinline__ uint64_t sat_add(uint64_t a, int64_t d) {
@@ -269,8 +324,169 @@ struct LineStats {
   unsigned long long first;  // min (line << 1 | has_strand) over records
 };
 
+// The fields of a record line.
+struct Fields {
+  uint64_t start, end;
+  int64_t bc_off;
+  uint32_t chrom_len, bc_len, count, strand;  // strand: 0 none, 1 '+', 2 '-'
+};
+
+// Eight characters whose first 8 - n stand before the field: their value as a
+// decimal number, or false if one of the last n (1 to 8) is no digit.
+__device__ __forceinline__ bool digits8(uint64_t w, uint32_t n, uint32_t* value) {
+  const uint64_t pad = n == 8 ? 0 : ~0ull >> (8 * n);  // bytes before the field
+  w = (w & ~pad) | (0x3030303030303030ull & pad);
+  const uint32_t a = (uint32_t)w ^ 0x30303030u, b = (uint32_t)(w >> 32) ^ 0x30303030u;  // 0 to 9 each, if digits
+  // a byte of 10 to 15 carries into its high half when 6 is added
+  if (((a | (a + 0x06060606u) | b | (b + 0x06060606u)) & 0xF0F0F0F0u) != 0) return false;
+  const uint32_t hi = __builtin_amdgcn_udot4(a, 0x0000010Au, 0u, false) * 100u + __builtin_amdgcn_udot4(a, 0x010A0000u, 0u, false);
+  const uint32_t lo = __builtin_amdgcn_udot4(b, 0x0000010Au, 0u, false) * 100u + __builtin_amdgcn_udot4(b, 0x010A0000u, 0u, false);
+  *value = hi * 10000u + lo;
+  return true;
+}
+
+// The number in the n characters that end before offset p.
+__device__ __forceinline__ bool digits(const NearText& t, int64_t p, uint32_t n, uint64_t* value) {
+  if (n == 0 || n > 16) return false;
+  uint32_t lo, hi = 0;
+  if (!digits8(t.at(p - 8), n < 8 ? n : 8, &lo)) return false;
+  if (n > 8 && !digits8(t.at(p - 16), n - 8, &hi)) return false;
+  *value = (uint64_t)hi * 100000000ull + lo;
+  return true;
+}
+
+// The fields of an ordinary record line [s, e) of staged text: at least four fields,
+// at most 64 characters, numbers of digits. The tabs come as one 64-bit mask from
+// the aligned words that hold the line, each number from the eight characters before
+// its end. False: the line goes through parse_fields (comments, errors, '.' fields,
+// long lines).
+__device__ __forceinline__ bool quick_fields(const NearText& t, int64_t s, int64_t e, Fields& f) {
+  const int len = (int)min<int64_t>(e - s, 65);
+  if (len < 7 || len > 64) return false;
+  const uint32_t r = (uint32_t)(s - t.first), skip = r & 3;
+  const uint32_t* w = t.w + (r >> 2);
+  if ((uint8_t)(w[0] >> (8 * skip)) == '#') return false;
+  uint64_t tabs = 0;
+  uint32_t over = 0;
+#pragma unroll
+  for (int k = 0; k < 17; k += 2) {
+    if (4 * k < len + (int)skip) {
+      uint32_t m[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const uint32_t x = (k + h < 17 ? w[k + h] : 0) ^ 0x09090909u;
+        const uint32_t y = (x & 0x7F7F7F7Fu) + 0x7F7F7F7Fu;
+        m[h] = (~(y | x) & 0x80808080u) >> 7;  // 1 in each byte that is a tab
+      }
+      const uint32_t bits = __builtin_amdgcn_udot4(m[1], 0x80402010u, __builtin_amdgcn_udot4(m[0], 0x08040201u, 0u, false), false);
+      if (k < 16) tabs |= (uint64_t)bits << (4 * k);
+      else over = bits;
+    }
+  }
+  tabs >>= skip;
+  if (skip) tabs |= (uint64_t)over << (64 - skip);
+  tabs &= ~0ull >> (64 - len);
+  if (popc64(tabs) < 3) return false;
+  const int t1 = lowbit64(tabs);
+  tabs &= tabs - 1;
+  const int t2 = lowbit64(tabs);
+  tabs &= tabs - 1;
+  const int t3 = lowbit64(tabs);
+  tabs &= tabs - 1;
+  const int t4 = tabs ? lowbit64(tabs) : len;
+  f.chrom_len = t1;
+  f.bc_off = s + t3 + 1;
+  f.bc_len = t4 - t3 - 1;
+  if (t1 == 0 || f.bc_len < 2) return false;
+  if (!digits(t, s + t2, t2 - t1 - 1, &f.start) || !digits(t, s + t3, t3 - t2 - 1, &f.end)) return false;
+  f.count = 1;
+  f.strand = 0;
+  if (tabs) {
+    tabs &= tabs - 1;
+    const int t5 = tabs ? lowbit64(tabs) : len;
+    uint64_t v;
+    if (t5 - t4 - 1 > 8 || !digits(t, s + t5, t5 - t4 - 1, &v)) return false;
+    f.count = (uint32_t)v;
+    if (tabs) {
+      tabs &= tabs - 1;
+      const int t6 = tabs ? lowbit64(tabs) : len;
+      const uint32_t c = (uint32_t)t.at(s + t5 + 1) & 255u;
+      if (t6 - t5 - 1 != 1 || (c != '+' && c != '-')) return false;
+      f.strand = c == '+' ? 1 : 2;
+    }
+  }
+  return true;
+}
+
+// The fields of any record line, one character after the other; an E_ code or 0.
+__device__ __forceinline__ uint32_t parse_fields(const uint8_t* __restrict__ text, int64_t n_bytes, int64_t s, int64_t e,
+                                              Fields& f, uint32_t& bc_c0) {
+  // current field
+  uint32_t field = 0, flen = 0, c0 = 0;
+  uint64_t num = 0;
+  bool nondigit = false;
+  int64_t fstart = s;
+  bool start_bad = false, end_bad = false, count_bad = false, strand_bad = false;
+  f = Fields{0, 0, s, 0, 0, 1, 0};
+  bc_c0 = 0;
+  int64_t a = s & ~(int64_t)7;
+  uint64_t word = load_word(text, a, n_bytes);
+  for (int64_t p = s; p <= e; ++p) {
+    uint32_t c = '\t';
+    if (p < e) {
+      if ((p & ~(int64_t)7) != a) {
+        a = p & ~(int64_t)7;
+        word = load_word(text, a, n_bytes);
+      }
+      c = (uint32_t)(word >> (8 * (p & 7))) & 0xFFu;
+    }
+    if (c == '\t') {
+      const bool bad = nondigit || flen == 0;
+      switch (field) {
+        case 0: f.chrom_len = flen; break;
+        case 1: f.start = num; start_bad = bad; break;
+        case 2: f.end = num; end_bad = bad; break;
+        case 3: f.bc_off = fstart; f.bc_len = flen; bc_c0 = c0; break;
+        case 4:
+          if (flen == 1 && c0 == '.') f.count = 1;
+          else { f.count = (uint32_t)num; count_bad = bad || num > 0xFFFFFFFFull; }
+          break;
+        case 5:
+          if (flen == 1 && c0 == '.') f.strand = 0;
+          else if (flen == 1 && c0 == '+') f.strand = 1;
+          else if (flen == 1 && c0 == '-') f.strand = 2;
+          else strand_bad = true;
+          break;
+        default: break;
+      }
+      ++field;
+      flen = 0;
+      num = 0;
+      nondigit = false;
+      fstart = p + 1;
+    } else {
+      const uint32_t d = c - '0';
+      const bool dig = d < 10;
+      const bool ovf = num > 1844674407370955161ull || (num == 1844674407370955161ull && d > 5);
+      nondigit |= !dig || ovf;
+      num = num * 10 + (dig ? d : 0);
+      c0 = flen == 0 ? c : c0;
+      ++flen;
+    }
+  }
+  if (field < 2) return E_START_MISSING;
+  if (start_bad) return E_START_BAD;
+  if (field < 3) return E_END_MISSING;
+  if (end_bad) return E_END_BAD;
+  if (field < 4) return E_BARCODE_MISSING;
+  if (count_bad) return E_COUNT_BAD;
+  if (strand_bad) return E_STRAND_BAD;
+  return 0;
+}
+
 // Parses line i and writes its record; accumulates the block statistics.
-__device__ __forceinline__ void parse_line(const uint8_t* __restrict__ text, int64_t n_bytes,
+template <typename Text>
+__device__ __forceinline__ void parse_line(const Text& t, const uint8_t* __restrict__ text, int64_t n_bytes,
                                            const int64_t* __restrict__ line_start, int64_t i,
                                            const uint8_t* __restrict__ chroms, int64_t shift_left,
                                            int64_t shift_right, const ParseOut& out, Counters* cnt,
@@ -281,109 +497,52 @@ __device__ __forceinline__ void parse_line(const uint8_t* __restrict__ text, int
     const int64_t s = line_start[i];
     int64_t e = line_start[i + 1] - 1;
     if (e > n_bytes) e = n_bytes;
-    if (e > s && load_byte(text, e - 1) == '\r') --e;
+    if (e > s && (t.at(e - 1) & 255) == '\r') --e;
     uint8_t fl = 0;
     uint32_t pos = 0, size = 0, count = 1;
     uint64_t bcw = 0, bch = 0;
-    const bool comment = e > s && load_byte(text, s) == '#';
-    if (e > s && !comment) {
+    Fields f{0, 0, s, 0, 0, 1, 0};
+    uint32_t bc_c0 = 0;
+    bool rec = false;
+    if constexpr (std::is_same_v<Text, NearText>) rec = quick_fields(t, s, e, f);
+    if (!rec && e > s && load_byte(text, s) != '#') {
+      rec = true;
+      err = parse_fields(text, n_bytes, s, e, f, bc_c0);
+    }
+    if (rec) {
       is_rec = true;
-      // current field
-      uint32_t field = 0, flen = 0, c0 = 0;
-      uint64_t num = 0, h = kFnvOffset;
-      bool nondigit = false;
-      int64_t fstart = s;
-      // committed fields
-      uint64_t chrom_h = 0, bc_h = 0, start = 0, end = 0;
-      int64_t chrom_off = s, bc_off = s;
-      uint32_t chrom_len = 0, bc_len = 0, bc_c0 = 0;
-      bool start_bad = false, end_bad = false, count_bad = false, strand_bad = false;
-      uint32_t strand = 0;  // 0 none, 1 '+', 2 '-'
-      int64_t a = s & ~(int64_t)7;
-      uint64_t word = load_word(text, a, n_bytes);
-      for (int64_t p = s; p <= e; ++p) {
-        uint32_t c = '\t';
-        if (p < e) {
-          if ((p & ~(int64_t)7) != a) {
-            a = p & ~(int64_t)7;
-            word = load_word(text, a, n_bytes);
-          }
-          c = (uint32_t)(word >> (8 * (p & 7))) & 0xFFu;
-        }
-        if (c == '\t') {
-          const bool bad = nondigit || flen == 0;
-          switch (field) {
-            case 0: chrom_h = h; chrom_off = fstart; chrom_len = flen; break;
-            case 1: start = num; start_bad = bad; break;
-            case 2: end = num; end_bad = bad; break;
-            case 3: bc_h = h; bc_off = fstart; bc_len = flen; bc_c0 = c0; break;
-            case 4:
-              if (flen == 1 && c0 == '.') count = 1;
-              else { count = (uint32_t)num; count_bad = bad || num > 0xFFFFFFFFull; }
-              break;
-            case 5:
-              if (flen == 1 && c0 == '.') strand = 0;
-              else if (flen == 1 && c0 == '+') strand = 1;
-              else if (flen == 1 && c0 == '-') strand = 2;
-              else strand_bad = true;
-              break;
-            default: break;
-          }
-          ++field;
-          flen = 0;
-          num = 0;
-          nondigit = false;
-          h = kFnvOffset;
-          fstart = p + 1;
-        } else {
-          const uint32_t d = c - '0';
-          const bool dig = d < 10;
-          const bool ovf = num > 1844674407370955161ull || (num == 1844674407370955161ull && d > 5);
-          nondigit |= !dig || ovf;
-          num = num * 10 + (dig ? d : 0);
-          h = fnv_step(h, c);
-          c0 = flen == 0 ? c : c0;
-          ++flen;
-        }
-      }
-      has_strand = strand != 0;  // a '.' strand field is no strand (qc.rs:338-344)
-      if (field < 2) err = E_START_MISSING;
-      else if (start_bad) err = E_START_BAD;
-      else if (field < 3) err = E_END_MISSING;
-      else if (end_bad) err = E_END_BAD;
-      else if (field < 4) err = E_BARCODE_MISSING;
-      else if (count_bad) err = E_COUNT_BAD;
-      else if (strand_bad) err = E_STRAND_BAD;
+      count = f.count;
+      has_strand = f.strand != 0;  // a '.' strand field is no strand (qc.rs:338-344)
       if (err == 0) {
         // shift_fragment (preprocessing.rs:173-183)
-        const uint64_t st = shift_left != 0 ? sat_add(start, shift_left) : start;
-        uint64_t en = end;
-        if (has_strand && shift_left != 0) en = sat_add(end, shift_left);
-        if (!has_strand && shift_right != 0) en = sat_add(end, shift_right);
+        const uint64_t st = shift_left != 0 ? sat_add(f.start, shift_left) : f.start;
+        uint64_t en = f.end;
+        if (has_strand && shift_left != 0) en = sat_add(f.end, shift_left);
+        if (!has_strand && shift_right != 0) en = sat_add(f.end, shift_right);
         if (en < st) {
           err = E_END_BEFORE_START;
         } else if (en > st) {
           fl |= F_KEEP;
-          if (bc_len == 1 && bc_c0 == '.') err = E_BARCODE_NONE;
-          else if (bc_len > 255) err = E_BARCODE_LONG;
-          bc_len_keep = bc_len;
+          if (f.bc_len == 1 && bc_c0 == '.') err = E_BARCODE_NONE;
+          else if (f.bc_len > 255) err = E_BARCODE_LONG;
+          bc_len_keep = f.bc_len;
           if (has_strand) fl |= F_STRAND;
-          if (strand == 2) fl |= F_REV;
+          if (f.strand == 2) fl |= F_REV;
           const uint64_t sz = en - st;
           size = (uint32_t)sz;
           if (sz > 0xFFFFFFFFull) fl |= F_HUGE;
-          if (sz > (strand == 2 ? 2147483648ull : 2147483647ull)) fl |= F_BIG;
-          const int ci = table_find(chroms, chrom_h, text + chrom_off, chrom_len);
+          if (sz > (f.strand == 2 ? 2147483648ull : 2147483647ull)) fl |= F_BIG;
+          const int ci = table_find(chroms, hash_text(t, s, f.chrom_len), t, s, f.chrom_len);
           if (ci >= 0) {
             const TableEntry& ce = table_entry(chroms, ci);
             fl |= F_GENOME;
             if (ce.flags & 1u) fl |= F_MITO;
-            const uint64_t coord = strand == 2 ? en - 1 : st;
+            const uint64_t coord = f.strand == 2 ? en - 1 : st;
             if (coord >= ce.length) fl |= F_RANGE;
             else pos = (uint32_t)(ce.base + coord);
           }
-          bcw = ((uint64_t)bc_off << 8) | (bc_len > 255 ? 255u : bc_len);
-          bch = bc_h;
+          bcw = ((uint64_t)f.bc_off << 8) | (f.bc_len > 255 ? 255u : f.bc_len);
+          if (err == 0) bch = hash_text(t, f.bc_off, f.bc_len);
         }
       }
     }
@@ -408,6 +567,14 @@ __device__ __forceinline__ void parse_line(const uint8_t* __restrict__ text, int
   ls.max_bc = bc_len_keep > ls.max_bc ? bc_len_keep : ls.max_bc;
 }
 
+// The text of a round's 256 lines is read once, in order, into LDS (kStage bytes; 16
+// below it and kStagePad above are read past a line's ends and masked away): a lane
+// reads its line in some thirty pieces, and from global memory those went to L2 again
+// and again (2.94 ms for 55 million lines of 41 characters that way, 1.99 ms staged;
+// 4.13 ms one character after the other, 0.9 ms the copy of the bytes alone). Rounds of longer lines read
+// the text where it lies, one character after the other.
+constexpr int kStage = 16384, kStagePad = 96;
+
 // kLineBlock lines per block (lane t of round r takes line b0 + r * 256 + t);
 // blk[block] = records kept. The block statistics go to the counters with one
 // atomic each, so the counters see a few tens of thousands of atomics.
@@ -417,12 +584,25 @@ __global__ void __launch_bounds__(kThreads) parse_kernel(const uint8_t* __restri
                                                          int64_t shift_right, ParseOut out, Counters* cnt,
                                                          int64_t* __restrict__ blk) {
   __shared__ unsigned long long red[6][kThreads / 64];
+  __shared__ uint4 stage[1 + kStage / 16 + kStagePad / 16];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int64_t b0 = (int64_t)blockIdx.x * kLineBlock;
   LineStats ls{0, 0, 0, 0, 0, ~0ull};
   for (int r = 0; r < kRounds; ++r) {
-    const int64_t i = b0 + (int64_t)r * kThreads + threadIdx.x;
-    if (i < n_lines) parse_line(text, n_bytes, line_start, i, chroms, shift_left, shift_right, out, cnt, ls);
+    const int64_t i0 = b0 + (int64_t)r * kThreads, i = i0 + threadIdx.x;
+    if (i0 >= n_lines) break;
+    const int64_t w0 = line_start[i0] / 16;
+    const int64_t stop = min(n_bytes, line_start[min(i0 + kThreads, n_lines)]);
+    if (stop - 16 * w0 <= kStage) {
+      for (int64_t w = w0 + threadIdx.x; 16 * w < stop; w += kThreads) stage[1 + w - w0] = load16(text, w, n_bytes);
+      __syncthreads();
+      if (i < n_lines)
+        parse_line(NearText{reinterpret_cast<const uint32_t*>(stage), 16 * w0 - 16}, text, n_bytes, line_start, i,
+                   chroms, shift_left, shift_right, out, cnt, ls);
+      __syncthreads();
+    } else if (i < n_lines) {
+      parse_line(FarText{text, n_bytes}, text, n_bytes, line_start, i, chroms, shift_left, shift_right, out, cnt, ls);
+    }
   }
   unsigned long long v[6] = {ls.n_rec, ls.n_strand, ls.n_keep, ls.max_bc, ls.first, ls.max_size};
 #pragma unroll
@@ -489,15 +669,6 @@ __global__ void __launch_bounds__(kThreads) keep_write_kernel(const uint8_t* __r
 // ---------------------------------------------------------------------------
 // 4. sort keys and barcode comparisons
 // ---------------------------------------------------------------------------
-
-// 8 bytes starting at byte p (any alignment) from two aligned loads.
-__device__ __forceinline__ uint64_t load_u8x8(const uint8_t* t, int64_t p, int64_t n) {
-  const int64_t a = p & ~(int64_t)7;
-  const int sh = (int)(p & 7) * 8;
-  const uint64_t lo = load_word(t, a, n);
-  if (sh == 0) return lo;
-  return (lo >> sh) | (load_word(t, a + 8, n) << (64 - sh));
-}
 
 // Equality of the len bytes at offsets a and b, eight at a time.
 __device__ __forceinline__ bool text_equal(const uint8_t* t, int64_t n, int64_t a, int64_t b, uint32_t len) {
@@ -650,7 +821,8 @@ __global__ void bad_group_kernel(const unsigned int* __restrict__ g_bad, const u
 }
 
 // Whitelist membership of each group's barcode (import.rs:74).
-__global__ void whitelist_kernel(const uint8_t* __restrict__ text, const uint32_t* __restrict__ gline,
+__global__ void whitelist_kernel(const uint8_t* __restrict__ text, int64_t n_bytes,
+                                 const uint32_t* __restrict__ gline,
                                  const uint64_t* __restrict__ bc, const uint64_t* __restrict__ bch,
                                  int64_t n_groups, const uint8_t* __restrict__ wl_table, uint8_t* __restrict__ wl) {
   const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -659,7 +831,7 @@ __global__ void whitelist_kernel(const uint8_t* __restrict__ text, const uint32_
   if (wl_table) {
     const uint32_t line = gline[g];
     const uint64_t b = bc[line];
-    w = table_find(wl_table, bch[line], text + (b >> 8), (uint32_t)(b & 255)) >= 0 ? 1 : 0;
+    w = table_find(wl_table, bch[line], FarText{text, n_bytes}, (int64_t)(b >> 8), (uint32_t)(b & 255)) >= 0 ? 1 : 0;
   }
   wl[g] = w;
 }
@@ -674,7 +846,7 @@ __global__ void group_hash_kernel(const uint32_t* __restrict__ gline, const uint
 
 // A barcode in two runs of sorted input (import.rs:139-141), among
 // whitelisted groups: equal hashes next to each other after sorting by hash.
-__global__ void dup_kernel(const uint8_t* __restrict__ text, const uint64_t* __restrict__ key,
+__global__ void dup_kernel(const uint8_t* __restrict__ text, int64_t n_bytes, const uint64_t* __restrict__ key,
                            const uint32_t* __restrict__ idx, const uint32_t* __restrict__ gline,
                            const uint64_t* __restrict__ bc, const uint8_t* __restrict__ wl, int64_t n_groups,
                            Counters* cnt) {
@@ -688,7 +860,8 @@ __global__ void dup_kernel(const uint8_t* __restrict__ text, const uint64_t* __r
     const uint32_t h = idx[q];
     if (!wl[h]) continue;
     const uint64_t c = bc[gline[h]];
-    if ((b & 255) == (c & 255) && bytes_equal(text + (b >> 8), text + (c >> 8), (uint32_t)(b & 255))) {
+    if ((b & 255) == (c & 255) &&
+        text_equal(text, n_bytes, (int64_t)(b >> 8), (int64_t)(c >> 8), (uint32_t)(b & 255))) {
       atomicMin(&cnt->dup, (unsigned long long)(g > h ? g : h));
       return;
     }
@@ -1052,9 +1225,13 @@ int data_error(unsigned long long word) {
 }
 
 uint64_t host_hash(const char* s, size_t len) {
-  uint64_t h = kFnvOffset;
-  for (size_t k = 0; k < len; ++k) h = fnv_step(h, (uint8_t)s[k]);
-  return h;
+  uint64_t h = hash_start((uint32_t)len);
+  for (size_t k = 0; k < len; k += 8) {
+    uint64_t w = 0;
+    memcpy(&w, s + k, len - k < 8 ? len - k : 8);
+    h = hash_step(h, w);
+  }
+  return hash_end(h);
 }
 
 }  // namespace frag
@@ -1071,7 +1248,7 @@ int64_t snapgpu_frag_table_bytes(const char* const* names, int32_t n) {
   while (cap < 2u * (uint32_t)n) cap <<= 1;
   int64_t bytes = (int64_t)sizeof(TableHeader) + (int64_t)cap * sizeof(TableSlot) + (int64_t)n * sizeof(TableEntry);
   for (int32_t k = 0; k < n; ++k) bytes += (int64_t)strlen(names[k]);
-  return bytes;
+  return bytes + kNamePad;
 }
 
 int snapgpu_frag_table_pack(const char* const* names, const uint64_t* lengths, const uint8_t* mito, int32_t n,
@@ -1329,7 +1506,7 @@ int snapgpu_frag_index(const uint8_t* d_text, int64_t n_bytes, int64_t n_lines, 
                                                    guniq, gbad);
   SG_LAUNCH_CHECK();
   uint8_t* wl = at<uint8_t>(w, Lo.wl);
-  whitelist_kernel<<<grid(G), kThreads, 0, st>>>(d_text, gline, po.bc, po.bch, G,
+  whitelist_kernel<<<grid(G), kThreads, 0, st>>>(d_text, n_bytes, gline, po.bc, po.bch, G,
                                                  static_cast<const uint8_t*>(d_whitelist), wl);
   SG_LAUNCH_CHECK();
   uint32_t* ordA = at<uint32_t>(w, Lo.ordA);
@@ -1342,7 +1519,7 @@ int snapgpu_frag_index(const uint8_t* d_text, int64_t n_bytes, int64_t n_lines, 
     hipcub::DoubleBuffer<uint64_t> gk(gkA, gkB);
     hipcub::DoubleBuffer<uint32_t> go(ordA, ordB);
     SG_HIP(hipcub::DeviceRadixSort::SortPairs(tmp, tmp_bytes, gk, go, (int)G, 0, 64, st));
-    dup_kernel<<<grid(G), kThreads, 0, st>>>(d_text, gk.Current(), go.Current(), gline, po.bc, wl, G, C);
+    dup_kernel<<<grid(G), kThreads, 0, st>>>(d_text, n_bytes, gk.Current(), go.Current(), gline, po.bc, wl, G, C);
     SG_LAUNCH_CHECK();
   }
   bad_group_kernel<<<grid(G), kThreads, 0, st>>>(gbad, wl, G, paired, C);

@@ -1,0 +1,92 @@
+"""Where the fragment import changes its way: lines at the limits of the eight-character
+parser (field lengths around 8 and 16 digits, lines around 64 characters, next to either
+end of the text, every optional field), and sort keys of just 64 bits and just more (group,
+position and value in one key or in two sorts), against the oracle, bit for bit."""
+import numpy as np
+import pytest
+
+from oracle.fragments import import_text
+from test_import_gpu import _check
+
+pytestmark = pytest.mark.gpu
+
+BIG = {"chr1": 2**32 - 1}
+
+
+def _gpu(text, sizes, **kw):
+    from snapatac2_amd.pp import import_fragment_text
+    return import_fragment_text(text, sizes, **kw)
+
+
+FORMS = [b"chr1\t%d\t%d\tAC" % (10**k, 10**k + 7) for k in range(10)]  # 1 to 10 digits
+FORMS += [b"chr1\t" + b"%d".rjust(2, b"0") % 3 + b"\t%s\tACGT-1" % (b"0" * z + b"99") for z in (0, 5, 6, 7, 13, 14, 15, 18)]
+FORMS += [b"chr1\t1\t9\t" + b"ACGT-" * 14 + b"A" * z for z in range(0, 3)]  # longer than 64
+FORMS += [(b"chr1\t1\t9\t" + b"G" * 80)[:n] for n in (12, 13, 61, 62, 63, 64, 65, 66, 72)]  # barcodes up to the line's end
+FORMS += [b"chr1\t1\t9\tAC\t%s" % c for c in (b"0", b"1", b".", b"99999999", b"4294967295", b"00000000005")]
+FORMS += [b"chr1\t1\t9\tAC\t2\t%s" % c for c in (b".",)] + [b"chr1\t5\t9\tAC\t2\t.\textra\tmore"]
+FORMS += [b"nochr\t1\t9\tAC", b"#chr1\t1\t9\tAC", b"", b"chr1\t7\t7\tAC", b"chr1\t1\t9\tA", b"chr1\t1\t9\t", b"\t1\t9\tAC",
+          b"chr1\t1\t9\tAC\r", b"chr1\t1\t9\tAC\t3\r", b"chr12345678\t1\t9\tAC"]
+STRANDED = [b"chr1\t1\t9\tAC\t2\t%s" % c for c in (b"+", b"-")] + [b"chr1\t1\t9\tAC\t.\t-\tx", b"chr1\t99999999\t100000007\tACGT\t1\t+"]
+
+
+@pytest.mark.parametrize("sorted_bc", [True, False])
+@pytest.mark.parametrize("fill", [0, 1, 40])
+def test_line_forms(torch_gpu, fill, sorted_bc):
+    """Every form between `fill` ordinary lines on either side: alone, the line is next to
+    both ends of the text, where the loads of eight characters don't fit."""
+    for forms, other in ((FORMS, b"chr1\t100\t250\tZZZZ\t1"), (STRANDED, b"chr1\t100\t250\tZZZZ\t1\t+")):
+        for form in forms:
+            for last in (b"\n", b""):
+                text = (other + b"\n") * fill + form + b"\n" + (other.replace(b"ZZZZ", b"zzzz") + b"\n") * fill
+                text = text[:-1] + last
+                print(fill, form, last, flush=True)
+                kw = dict(min_num_fragments=0, sorted_by_barcode=sorted_bc)
+                _check(_gpu(text, BIG, **kw), import_text(text, BIG, **kw))
+
+
+def _bits(x):
+    return max(int(x).bit_length(), 1)
+
+
+# (genome length, largest size, barcodes): key bits without the mark of unsorted input
+KEYS = [(2**30 - 1, 2**29 - 1, 16), (2**30 - 1, 2**30 - 1, 16), (2**30 - 1, 2**31 - 1, 16), (2**30 - 1, 2**31 - 1, 17),
+        (2**32 - 1, 2**32 - 1, 1), (2**32 - 1, 2**32 - 1, 2), (2**32 - 1, 2**31 - 1, 1), (2**20, 600, 1), (2**20, 600, 300)]
+
+
+@pytest.mark.parametrize("total,size,n_bc", KEYS)
+@pytest.mark.parametrize("sorted_bc", [True, False])
+@pytest.mark.parametrize("single", [False, True])
+def test_key_widths(torch_gpu, total, size, n_bc, sorted_bc, single):
+    rng = np.random.default_rng(n_bc + size % 1000)
+    if single:
+        size = min(size // 2, 2**31 - 1)
+    sizes = {"chrM": 1000, "chr1": total - 1000}
+    n = 3000
+    lines = []
+    for i in range(n):
+        chrom = ("chr1", "chr1", "chr1", "chrM", "chrU")[int(rng.integers(5))]
+        ln = size if i == 7 else int(rng.integers(1, min(size, 500) + 1))
+        start = 900 if i == 7 else int(rng.integers(0, 500 if chrom == "chrM" else total - 1000 - 600))
+        if i == 7:
+            chrom = "chr1"
+        # a '-' record is stored by its last base, which has to lie in the chromosome
+        strand = "\t" + ("-" if rng.random() < 0.5 and i != 7 else "+") if single else ""
+        lines.append((f"bc{int(rng.integers(n_bc)):03d}x", f"{chrom}\t{start}\t{start + ln}\t", f"\t{int(rng.integers(1, 4))}{strand}"))
+    if sorted_bc:
+        lines.sort(key=lambda t: t[0])
+    text = "\n".join(a + b + c for b, a, c in lines).encode()
+    kw = dict(min_num_fragments=0, sorted_by_barcode=sorted_bc)
+    ref = import_text(text, sizes, **kw)
+    assert len(ref["barcodes"]) == min(n_bc, len(ref["barcodes"])) > 0
+    _check(_gpu(text, sizes, **kw), ref)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 5000])
+@pytest.mark.parametrize("distinct", [True, False])
+def test_groups_of_unsorted_lines(torch_gpu, n, distinct):
+    """All barcodes different (the table at its fullest), or all records of one."""
+    rng = np.random.default_rng(n)
+    ids = rng.permutation(n) if distinct else np.zeros(n, int)
+    text = b"".join(b"chr1\t%d\t%d\tcell%d\t%d\n" % (s, s + 50, i, 1 + s % 3) for i, s in zip(ids, rng.integers(0, 900, n)))
+    kw = dict(min_num_fragments=0, sorted_by_barcode=False)
+    _check(_gpu(text, {"chr1": 1000}, **kw), import_text(text, {"chr1": 1000}, **kw))
