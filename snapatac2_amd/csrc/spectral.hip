@@ -1001,7 +1001,9 @@ static void launch_vjp(const int64_t* indptr, const int32_t* idx, const uint32_t
     }
     if constexpr (BW == 16) {
       if (over) {
-        window::product16_scaled(*over->csr_windows, dense, nullptr, out, st);
+        // (the pair sums of the CSC product have been read)
+        window::product16_scaled(*over->csr_windows, dense, nullptr, out, over->partial, over->csc->n_pairs,
+                                 st);
         return;
       }
     }

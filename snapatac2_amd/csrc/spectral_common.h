@@ -78,8 +78,8 @@ void product32_scaled(const snapgpu_panel_layout& L, const float* dense, float* 
 
 namespace window {
 // The same over the window layout (window.hip): the CSR product of the adjoint over
-// the mixed layout.
-void product16_scaled(const snapgpu_window_layout& L, const float* dense, const float* scale, float* out,
-                      hipStream_t st);
+// the mixed layout. spare: spare_rows rows of 16 floats that may be overwritten.
+void product16_scaled(const snapgpu_window_layout& L, const float* dense, const float* scale, float* out, float* spare,
+                      int64_t spare_rows, hipStream_t st);
 }  // namespace window
 }  // namespace snapgpu

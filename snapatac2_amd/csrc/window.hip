@@ -49,6 +49,10 @@ constexpr int kChunk = 64;                         // build chunk of a row
 constexpr int kThreads = 1024;
 constexpr int kQuads = kThreads / 4;
 constexpr int kMaxWindows = 16384;                 // LDS counters of the build (64 KB)
+#ifndef SNAPGPU_WINDOW_PRE
+#define SNAPGPU_WINDOW_PRE 16
+#define SNAPGPU_WINDOW_STEP 4
+#endif
 constexpr uint32_t kFlag = 1u << (kWinBits + 11);  // after the column and the 11-bit slot
 static_assert(kWinBits + 12 <= 24, "column, slot and flag must stay below the count byte");
 
@@ -222,7 +226,7 @@ __global__ void quad_split_kernel(const int64_t* __restrict__ bstart, const uint
 }
 
 // ---------------------------------------------------------------------------
-// The product. Workgroup b walks the windows; quad k sums its chunk's pieces
+// The product. A workgroup walks its block's windows; quad k sums its chunk's pieces
 // (4 lanes, lane j holding columns 4j..4j+3) and adds each piece to its slot;
 // a barrier closes each window. The epilogue adds each row's slots in order:
 //   EPI 0: out32[row][c] = scale[row] * sum (sum when scale is null) (FP32, stride 16)
@@ -254,124 +258,216 @@ __device__ __forceinline__ void gather_entry(float4* acc, int q, uint32_t v, con
   a.w = fmaf(x, z.w, a.w);
 }
 
+// The launch of a product: blocks [0, full) have a workgroup each, the others are
+// cut along their windows into kShares equal shares, one workgroup each, whose row
+// sums go to part (kSlots rows for each of a share's at most two blocks, a row at its
+// first slot; rows without entries have none) and are added in window order by
+// share_sum_kernel.
+constexpr int kShares = 256;  // the card's CUs: a workgroup's accumulators fill one
+
+__host__ __device__ inline int64_t share_start(int64_t k, int64_t n_blocks, int64_t nw) {
+  return k * (n_blocks * nw) / kShares;  // in windows of the cut blocks, one after the other
+}
+
+// Sum of a row's slots, in order.
+__device__ __forceinline__ float4 row_sum(const float4* acc, uint32_t rs, int q) {
+  const uint32_t s0 = rs & 0xFFFFu, ns = rs >> 16;
+  float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (uint32_t j = 0; j < ns; ++j) {
+    const float4 a = acc[(s0 + j) * 4 + q];
+    t.x += a.x;
+    t.y += a.y;
+    t.z += a.z;
+    t.w += a.w;
+  }
+  return t;
+}
+
+template <int EPI>
+__device__ __forceinline__ void store_row(float4 t, int64_t row, int q, const float* __restrict__ scale,
+                                          float* __restrict__ out32, const double* __restrict__ V, int64_t ldv,
+                                          const double* __restrict__ dinv, double* __restrict__ Y, int64_t ldy, int b) {
+  const float sc = scale ? scale[row] : 1.f;
+  const float o[4] = {t.x * sc, t.y * sc, t.z * sc, t.w * sc};
+  if (EPI == 0) {
+    *reinterpret_cast<float4*>(out32 + row * 16 + q * 4) = make_float4(o[0], o[1], o[2], o[3]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int c = q * 4 + j;
+      if (c < b) Y[row * ldy + c] = (double)o[j] - dinv[row] * V[row * ldv + c];
+    }
+  }
+}
+
 template <int EPI>
 __global__ void __launch_bounds__(kThreads) product_kernel(
     const uint32_t* __restrict__ ent, const int64_t* __restrict__ bstart, const uint32_t* __restrict__ qoff,
     int64_t nw, const int64_t* __restrict__ block_row, const uint32_t* __restrict__ row_slot,
     const float* __restrict__ dense, const float* __restrict__ scale, float* __restrict__ out32,
     const double* __restrict__ V, int64_t ldv, const double* __restrict__ dinv, double* __restrict__ Y,
-    int64_t ldy, int b) {
+    int64_t ldy, int b, int64_t full, int64_t n_blocks, float4* __restrict__ part) {
   __shared__ float4 acc[kSlots * 4];
   const int tid = threadIdx.x, quad = tid >> 2, q = tid & 3;
-  for (int i = tid; i < kSlots * 4; i += kThreads) acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-  __syncthreads();
-  const int64_t blk = blockIdx.x;
   const char* db = reinterpret_cast<const char*>(dense);
   const uint32_t q16 = (uint32_t)q << 4;
-  // Window w + 2's bounds and window w + 1's first 24 entries are loaded while
-  // window w is summed, so neither dependent load (bounds, then entries) sits
-  // on a window's critical path. Entries past a chunk's end read as 0 (no piece
-  // start, count 0): they add 0 * z to the open piece, z being a row of the
-  // same window.
-  constexpr int kPre = 24;
-  const int64_t bq0 = blk * nw;
-  int64_t bs = bstart[bq0];
-  uint32_t p0 = qoff[bq0 * (kQuads + 1) + quad], p1 = qoff[bq0 * (kQuads + 1) + quad + 1];
-  int64_t bs1 = 0;
-  uint32_t p01 = 0, p11 = 0;
-  if (nw > 1) {
-    bs1 = bstart[bq0 + 1];
-    p01 = qoff[(bq0 + 1) * (kQuads + 1) + quad];
-    p11 = qoff[(bq0 + 1) * (kQuads + 1) + quad + 1];
-  }
-  uint32_t vpre[kPre];
-#pragma unroll
-  for (int u = 0; u < kPre; ++u) vpre[u] = p0 + u < p1 ? ent[bs + p0 + u] : 0u;
-  for (int64_t w = 0; w < nw; ++w) {
-    const bool more1 = w + 1 < nw, more2 = w + 2 < nw;
-    // window w + 1's first entries, window w + 2's bounds
-    uint32_t vn[kPre];
-#pragma unroll
-    for (int u = 0; u < kPre; ++u) vn[u] = (more1 && p01 + u < p11) ? ent[bs1 + p01 + u] : 0u;
-    int64_t bs2 = 0;
-    uint32_t p02 = 0, p12 = 0;
-    if (more2) {
-      const int64_t bq2 = bq0 + w + 2;
-      bs2 = bstart[bq2];
-      p02 = qoff[bq2 * (kQuads + 1) + quad];
-      p12 = qoff[bq2 * (kQuads + 1) + quad + 1];
-    }
-    const uint32_t* eb = ent + bs;
-    const uint32_t wbase = ((uint32_t)w << (kWinBits + 6)) | q16;  // window w, this lane's 16 bytes
-    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
-    uint32_t slot = 0;
-    bool open = false;  // the chunk starts at a piece start, so its first entry opens one
-#pragma unroll
-    for (int h = 0; h < kPre; h += 8) {
-      if (p0 + h < p1) {
-        float4 z[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-          z[u] = *reinterpret_cast<const float4*>(db + (((vpre[h + u] & (uint32_t)(kWin - 1)) << 6) | wbase));
-#pragma unroll
-        for (int u = 0; u < 8; ++u) gather_entry(acc, q, vpre[h + u], z[u], open, slot, a);
-      }
-    }
-    for (uint32_t p = p0 + kPre; p < p1; p += 8) {
-      uint32_t v[8];
-      float4 z[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = p + u < p1 ? eb[p + u] : 0u;
-#pragma unroll
-      for (int u = 0; u < 8; ++u) z[u] = *reinterpret_cast<const float4*>(db + (((v[u] & (uint32_t)(kWin - 1)) << 6) | wbase));
-#pragma unroll
-      for (int u = 0; u < 8; ++u) gather_entry(acc, q, v[u], z[u], open, slot, a);
-    }
-    if (open) add_piece(acc, slot, q, a);
+  const bool whole = blockIdx.x < full;
+  const int64_t share = (int64_t)blockIdx.x - full;
+  int64_t at = whole ? 0 : share_start(share, n_blocks - full, nw);
+  const int64_t stop = whole ? nw : share_start(share + 1, n_blocks - full, nw);
+  for (int seg = 0; at < stop; ++seg) {
+    const int64_t blk = whole ? blockIdx.x : full + at / nw;
+    const int64_t w0 = whole ? 0 : at % nw;
+    const int64_t w1 = min(nw, w0 + (stop - at));
+    for (int i = tid; i < kSlots * 4; i += kThreads) acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     __syncthreads();
-    bs = bs1;
-    p0 = p01;
-    p1 = p11;
-    bs1 = bs2;
-    p01 = p02;
-    p11 = p12;
+    // Window w + 2's bounds and window w + 1's first kPre entries are loaded while
+    // window w is summed, so neither dependent load (bounds, then entries) sits
+    // on a window's critical path. Entries past a chunk's end read as 0 (no piece
+    // start, count 0): they add 0 * z to the open piece, z being a row of the
+    // same window. A quad's chunk is nine entries on average at 891 million
+    // entries in 778 blocks x 489 windows, so what is taken at once is small: per
+    // application 11.93 ms with 24 loaded ahead and 8 at a time, 11.71 with 16 and
+    // 8, 11.28 with 16 and 4, 11.39 with 8 and 4.
+    constexpr int kPre = SNAPGPU_WINDOW_PRE, kStep = SNAPGPU_WINDOW_STEP;
+    const int64_t bq0 = blk * nw;
+    int64_t bs = bstart[bq0 + w0];
+    uint32_t p0 = qoff[(bq0 + w0) * (kQuads + 1) + quad], p1 = qoff[(bq0 + w0) * (kQuads + 1) + quad + 1];
+    int64_t bs1 = 0;
+    uint32_t p01 = 0, p11 = 0;
+    if (w0 + 1 < w1) {
+      bs1 = bstart[bq0 + w0 + 1];
+      p01 = qoff[(bq0 + w0 + 1) * (kQuads + 1) + quad];
+      p11 = qoff[(bq0 + w0 + 1) * (kQuads + 1) + quad + 1];
+    }
+    uint32_t vpre[kPre];
 #pragma unroll
-    for (int u = 0; u < kPre; ++u) vpre[u] = vn[u];
+    for (int u = 0; u < kPre; ++u) vpre[u] = p0 + u < p1 ? ent[bs + p0 + u] : 0u;
+    for (int64_t w = w0; w < w1; ++w) {
+      const bool more1 = w + 1 < w1, more2 = w + 2 < w1;
+      // window w + 1's first entries, window w + 2's bounds
+      uint32_t vn[kPre];
+#pragma unroll
+      for (int u = 0; u < kPre; ++u) vn[u] = (more1 && p01 + u < p11) ? ent[bs1 + p01 + u] : 0u;
+      int64_t bs2 = 0;
+      uint32_t p02 = 0, p12 = 0;
+      if (more2) {
+        const int64_t bq2 = bq0 + w + 2;
+        bs2 = bstart[bq2];
+        p02 = qoff[bq2 * (kQuads + 1) + quad];
+        p12 = qoff[bq2 * (kQuads + 1) + quad + 1];
+      }
+      const uint32_t* eb = ent + bs;
+      const uint32_t wbase = ((uint32_t)w << (kWinBits + 6)) | q16;  // window w, this lane's 16 bytes
+      float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+      uint32_t slot = 0;
+      bool open = false;  // the chunk starts at a piece start, so its first entry opens one
+#pragma unroll
+      for (int h = 0; h < kPre; h += kStep) {
+        if (p0 + h < p1) {
+          float4 z[kStep];
+#pragma unroll
+          for (int u = 0; u < kStep; ++u)
+            z[u] = *reinterpret_cast<const float4*>(db + (((vpre[h + u] & (uint32_t)(kWin - 1)) << 6) | wbase));
+#pragma unroll
+          for (int u = 0; u < kStep; ++u) gather_entry(acc, q, vpre[h + u], z[u], open, slot, a);
+        }
+      }
+      for (uint32_t p = p0 + kPre; p < p1; p += kStep) {
+        uint32_t v[kStep];
+        float4 z[kStep];
+#pragma unroll
+        for (int u = 0; u < kStep; ++u) v[u] = p + u < p1 ? eb[p + u] : 0u;
+#pragma unroll
+        for (int u = 0; u < kStep; ++u)
+          z[u] = *reinterpret_cast<const float4*>(db + (((v[u] & (uint32_t)(kWin - 1)) << 6) | wbase));
+#pragma unroll
+        for (int u = 0; u < kStep; ++u) gather_entry(acc, q, v[u], z[u], open, slot, a);
+      }
+      if (open) add_piece(acc, slot, q, a);
+      __syncthreads();
+      bs = bs1;
+      p0 = p01;
+      p1 = p11;
+      bs1 = bs2;
+      p01 = p02;
+      p11 = p12;
+#pragma unroll
+      for (int u = 0; u < kPre; ++u) vpre[u] = vn[u];
+    }
+    // epilogue: 4 lanes per row
+    const int64_t r0 = block_row[blk], r1 = block_row[blk + 1];
+    for (int64_t row = r0 + quad; row < r1; row += kQuads) {
+      const uint32_t rs = row_slot[row];
+      const float4 t = row_sum(acc, rs, q);
+      if (whole) store_row<EPI>(t, row, q, scale, out32, V, ldv, dinv, Y, ldy, b);
+      else if (rs >> 16) part[((share * 2 + seg) * kSlots + (rs & 0xFFFFu)) * 4 + q] = t;
+    }
+    at += w1 - w0;
+    __syncthreads();
   }
-  // epilogue: 4 lanes per row
-  const int64_t r0 = block_row[blk], r1 = block_row[blk + 1];
-  for (int64_t row = r0 + quad; row < r1; row += kQuads) {
+}
+
+// The rows of cut block full + blockIdx.y: the sums of its shares, in window order.
+template <int EPI>
+__global__ void __launch_bounds__(256) share_sum_kernel(
+    int64_t nw, const int64_t* __restrict__ block_row, const uint32_t* __restrict__ row_slot,
+    const float* __restrict__ scale, float* __restrict__ out32, const double* __restrict__ V, int64_t ldv,
+    const double* __restrict__ dinv, double* __restrict__ Y, int64_t ldy, int b, int64_t full, int64_t n_blocks,
+    const float4* __restrict__ part) {
+  const int64_t cut = blockIdx.y, rest = n_blocks - full;
+  const int64_t r1 = block_row[full + cut + 1];
+  const int q = threadIdx.x & 3;
+  for (int64_t row = block_row[full + cut] + blockIdx.x * 64 + (threadIdx.x >> 2); row < r1; row += gridDim.x * 64) {
     const uint32_t rs = row_slot[row];
-    const uint32_t s0 = rs & 0xFFFFu, ns = rs >> 16;
     float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (uint32_t j = 0; j < ns; ++j) {
-      const float4 a = acc[(s0 + j) * 4 + q];
+    // shares that hold windows of [cut * nw, (cut + 1) * nw); none before the first k
+    // does, as share_start rounds down
+    for (int64_t k = max<int64_t>(0, cut * kShares / rest - 1); k < kShares && (rs >> 16); ++k) {
+      const int64_t u0 = share_start(k, rest, nw), u1 = share_start(k + 1, rest, nw);
+      if (u0 >= (cut + 1) * nw) break;
+      if (u1 <= cut * nw || u0 == u1) continue;
+      const float4 a = part[((k * 2 + (u0 >= cut * nw ? 0 : 1)) * kSlots + (rs & 0xFFFFu)) * 4 + q];
       t.x += a.x;
       t.y += a.y;
       t.z += a.z;
       t.w += a.w;
     }
-    const float sc = scale ? scale[row] : 1.f;
-    const float o[4] = {t.x * sc, t.y * sc, t.z * sc, t.w * sc};
-    if (EPI == 0) {
-      *reinterpret_cast<float4*>(out32 + row * 16 + q * 4) = make_float4(o[0], o[1], o[2], o[3]);
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int c = q * 4 + j;
-        if (c < b) Y[row * ldy + c] = (double)o[j] - dinv[row] * V[row * ldv + c];
-      }
-    }
+    store_row<EPI>(t, row, q, scale, out32, V, ldv, dinv, Y, ldy, b);
   }
+}
+
+// out32 / Y as the kernels' (EPI 0 / 1). spare: `spare_rows` rows of 16 floats that
+// may be overwritten, or null.
+//
+// A workgroup has a CU to itself, so n_blocks workgroups take ceil(n_blocks / 256)
+// turns and the last may leave most CUs idle: 778 blocks take four turns for the work
+// of 3.04. Where there is a whole turn before it and the last one is at most 7/8
+// full, its blocks are cut into shares instead (891 million entries in 778 blocks:
+// 13.56 -> 11.93 ms per application of both products).
+// With one turn or less the sums stay in one piece.
+template <int EPI>
+static void product(const snapgpu_window_layout& L, const float* dense, const float* scale, float* out32,
+                    const double* V, int64_t ldv, const double* dinv, double* Y, int64_t ldy, int b, float* spare,
+                    int64_t spare_rows, hipStream_t st) {
+  const int64_t rest = L.n_blocks % kShares;
+  const bool cut = L.n_blocks > kShares && rest > 0 && 8 * rest <= 7 * kShares && spare != nullptr &&
+                   spare_rows >= 2 * (int64_t)kShares * kSlots;
+  const int64_t full = cut ? L.n_blocks - rest : L.n_blocks;
+  float4* part = reinterpret_cast<float4*>(spare);
+  product_kernel<EPI><<<(unsigned)(full + (cut ? kShares : 0)), kThreads, 0, st>>>(
+      L.ent, L.bucket_start, L.quad_off, L.n_windows, L.block_row, L.row_slot, dense, scale, out32, V, ldv, dinv, Y,
+      ldy, b, full, L.n_blocks, part);
+  if (cut)
+    share_sum_kernel<EPI><<<dim3(kSlots / 64, (unsigned)rest), 256, 0, st>>>(
+        L.n_windows, L.block_row, L.row_slot, scale, out32, V, ldv, dinv, Y, ldy, b, full, L.n_blocks, part);
 }
 
 static int64_t align256(int64_t b) { return (b + 255) / 256 * 256; }
 
-void product16_scaled(const snapgpu_window_layout& L, const float* dense, const float* scale, float* out,
-                      hipStream_t st) {
-  product_kernel<0><<<(unsigned)L.n_blocks, kThreads, 0, st>>>(L.ent, L.bucket_start, L.quad_off, L.n_windows,
-                                                               L.block_row, L.row_slot, dense, scale, out, nullptr,
-                                                               0, nullptr, nullptr, 0, 16);
+void product16_scaled(const snapgpu_window_layout& L, const float* dense, const float* scale, float* out, float* spare,
+                      int64_t spare_rows, hipStream_t st) {
+  product<0>(L, dense, scale, out, nullptr, 0, nullptr, nullptr, 0, 16, spare, spare_rows, st);
 }
 
 struct PlanWs {
@@ -530,12 +626,8 @@ int snapgpu_spectral_apply_window(const snapgpu_window_layout* csr, const snapgp
   q += align256(n * 16 * 4);
   float* Z = (float*)q;
   scale_in_kernel<16><<<(unsigned)ceil_div(n * 16, 256), 256, 0, st>>>(d_V, ldv, n, b, d_r32, Vs);
-  product_kernel<0><<<(unsigned)csc->n_blocks, kThreads, 0, st>>>(
-      csc->ent, csc->bucket_start, csc->quad_off, csc->n_windows, csc->block_row, csc->row_slot, Vs, d_w2, Z,
-      nullptr, 0, nullptr, nullptr, 0, b);
-  product_kernel<1><<<(unsigned)csr->n_blocks, kThreads, 0, st>>>(
-      csr->ent, csr->bucket_start, csr->quad_off, csr->n_windows, csr->block_row, csr->row_slot, Z, d_r32,
-      nullptr, d_V, ldv, d_dinv, d_Y, ldy, b);
+  product<0>(*csc, Vs, d_w2, Z, nullptr, 0, nullptr, nullptr, 0, b, nullptr, 0, st);
+  product<1>(*csr, Z, d_r32, nullptr, d_V, ldv, d_dinv, d_Y, ldy, b, Vs, n, st);  // Vs has been read
   SG_LAUNCH_CHECK();
   return SNAPGPU_OK;
 }
@@ -566,9 +658,8 @@ int snapgpu_spectral_apply_mixed(const snapgpu_window_layout* csr, const snapgpu
   scale_in_kernel<16><<<(unsigned)ceil_div(n * 16, 256), 256, 0, st>>>(d_V, ldv, n, b, d_r32, Vs);
   // Z = w^2 o (X^T Vs) over the CSC panels, then Y = r o (X Z) - dinv o V over the CSR windows
   panel::product16_scaled(*csc, Vs, part, d_w2, Z, st);
-  product_kernel<1><<<(unsigned)csr->n_blocks, kThreads, 0, st>>>(
-      csr->ent, csr->bucket_start, csr->quad_off, csr->n_windows, csr->block_row, csr->row_slot, Z, d_r32,
-      nullptr, d_V, ldv, d_dinv, d_Y, ldy, b);
+  // (the pair sums have been read)
+  product<1>(*csr, Z, d_r32, nullptr, d_V, ldv, d_dinv, d_Y, ldy, b, part, csc->n_pairs, st);
   SG_LAUNCH_CHECK();
   return SNAPGPU_OK;
 }
