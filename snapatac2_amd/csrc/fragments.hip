@@ -501,15 +501,17 @@ __device__ __forceinline__ uint32_t parse_fields(const uint8_t* __restrict__ tex
   return 0;
 }
 
-// Parses line i and writes its record; accumulates the block statistics.
+// Parses line i and writes its record; accumulates the block statistics. Returns
+// the barcode (as in ParseOut) of a record that is kept, or 0.
 template <typename Text>
-__device__ __forceinline__ void parse_line(const Text& t, const uint8_t* __restrict__ text, int64_t n_bytes,
+__device__ __forceinline__ uint64_t parse_line(const Text& t, const uint8_t* __restrict__ text, int64_t n_bytes,
                                            const int64_t* __restrict__ line_start, int64_t i,
                                            const uint8_t* __restrict__ chroms, int64_t shift_left,
                                            int64_t shift_right, const ParseOut& out, Counters* cnt,
                                            LineStats& ls) {
   bool is_rec = false, has_strand = false;
   uint32_t err = 0, bc_len_keep = 0;
+  uint64_t kept = 0;
   {
     const int64_t s = line_start[i];
     int64_t e = line_start[i + 1] - 1;
@@ -571,6 +573,7 @@ __device__ __forceinline__ void parse_line(const Text& t, const uint8_t* __restr
     out.bch[i] = bch;
     if (err) atomicMin(&cnt->err, ((unsigned long long)i << 8) | err);
     if (!err && (fl & F_KEEP)) {
+      kept = bcw;
       ++ls.n_keep;
       ls.max_size = size > ls.max_size ? size : ls.max_size;
     }
@@ -582,6 +585,7 @@ __device__ __forceinline__ void parse_line(const Text& t, const uint8_t* __restr
     ls.first = f < ls.first ? f : ls.first;
   }
   ls.max_bc = bc_len_keep > ls.max_bc ? bc_len_keep : ls.max_bc;
+  return kept;
 }
 
 // The text of a round's 256 lines is read once, in order, into LDS (kStage bytes; 16
@@ -592,6 +596,9 @@ __device__ __forceinline__ void parse_line(const Text& t, const uint8_t* __restr
 // the text where it lies, one character after the other.
 constexpr int kStage = 16384, kStagePad = 96;
 
+// same[i] (input sorted by barcode, else null): 1 if this line and the one before
+// are kept and their barcodes are known to be equal (both were staged).
+//
 // kLineBlock lines per block (lane t of round r takes line b0 + r * 256 + t);
 // blk[block] = records kept. The block statistics go to the counters with one
 // atomic each, so the counters see a few tens of thousands of atomics.
@@ -599,9 +606,10 @@ __global__ void __launch_bounds__(kThreads) parse_kernel(const uint8_t* __restri
                                                          const int64_t* __restrict__ line_start, int64_t n_lines,
                                                          const uint8_t* __restrict__ chroms, int64_t shift_left,
                                                          int64_t shift_right, ParseOut out, Counters* cnt,
-                                                         int64_t* __restrict__ blk) {
+                                                         int64_t* __restrict__ blk, uint8_t* __restrict__ same) {
   __shared__ unsigned long long red[6][kThreads / 64];
   __shared__ uint4 stage[1 + kStage / 16 + kStagePad / 16];
+  __shared__ uint64_t barcode[kThreads];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int64_t b0 = (int64_t)blockIdx.x * kLineBlock;
   LineStats ls{0, 0, 0, 0, 0, ~0ull};
@@ -613,12 +621,28 @@ __global__ void __launch_bounds__(kThreads) parse_kernel(const uint8_t* __restri
     if (stop - 16 * w0 <= kStage) {
       for (int64_t w = w0 + threadIdx.x; 16 * w < stop; w += kThreads) stage[1 + w - w0] = load16(text, w, n_bytes);
       __syncthreads();
+      const NearText near{reinterpret_cast<const uint32_t*>(stage), 16 * w0 - 16};
+      uint64_t b = 0;
       if (i < n_lines)
-        parse_line(NearText{reinterpret_cast<const uint32_t*>(stage), 16 * w0 - 16}, text, n_bytes, line_start, i,
-                   chroms, shift_left, shift_right, out, cnt, ls);
+        b = parse_line(near, text, n_bytes, line_start, i, chroms, shift_left, shift_right, out, cnt, ls);
+      if (same) {
+        barcode[threadIdx.x] = b;
+        __syncthreads();
+        if (i < n_lines) {
+          const uint64_t p = threadIdx.x > 0 ? barcode[threadIdx.x - 1] : 0;
+          const uint32_t len = (uint32_t)(b & 255);
+          bool eq = b && p && (uint32_t)(p & 255) == len;
+          for (uint32_t k = 0; eq && k < len; k += 8) {
+            const uint64_t x = near.at((int64_t)(b >> 8) + k) ^ near.at((int64_t)(p >> 8) + k);
+            eq = (len - k < 8 ? first_bytes(x, len - k) : x) == 0;
+          }
+          same[i] = eq ? 1 : 0;
+        }
+      }
       __syncthreads();
     } else if (i < n_lines) {
       parse_line(FarText{text, n_bytes}, text, n_bytes, line_start, i, chroms, shift_left, shift_right, out, cnt, ls);
+      if (same) same[i] = 0;
     }
   }
   unsigned long long v[6] = {ls.n_rec, ls.n_strand, ls.n_keep, ls.max_bc, ls.first, ls.max_size};
@@ -714,43 +738,26 @@ __device__ __forceinline__ uint64_t pv_of(uint8_t f, uint32_t pos, uint32_t size
 }
 
 // Boundaries of equal-barcode runs over kept records in file order (input
-// sorted by barcode): run[v] = 1 where a new run starts. Each lane reads its own
-// barcode; the one before comes from the lane below. 55 million records: 1.46 ms
-// with both read by each lane, 0.91 ms so, which is the text's passage once more
-// (3.8 GB with the records).
+// sorted by barcode): run[v] = 1 where a new run starts. What the parser could not
+// tell from staged text (the first line of its rounds, after a line that was not kept)
+// is compared here. 55 million records: 0.91 ms with every barcode compared here (the
+// text once more), 0.39 so, and 0.1 more in the parser.
 __global__ void __launch_bounds__(kThreads) run_bound_kernel(const uint8_t* __restrict__ text, int64_t n_bytes,
                                                              const uint32_t* __restrict__ kept,
                                                              const uint64_t* __restrict__ bc,
-                                                             const uint64_t* __restrict__ bch, int64_t n,
+                                                             const uint8_t* __restrict__ same, int64_t n,
                                                              int64_t* __restrict__ run) {
   const int64_t v = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-  const int lane = threadIdx.x & 63, below = lane > 0 ? lane - 1 : 0;
-  const bool act = v < n;
-  uint64_t b = 0, h = 0, pb = 0, ph = 0;
-  if (act) {
-    const uint32_t line = kept[v];
-    b = bc[line];
-    h = bch[line];
+  const uint32_t line = v < n ? kept[v] : 0;
+  uint32_t before = (uint32_t)__shfl_up((int)line, 1, 64);
+  if (v >= n) return;
+  if ((threadIdx.x & 63) == 0) before = v > 0 ? kept[v - 1] : 0;
+  bool eq = v > 0 && line == before + 1 && same[line];
+  if (!eq && v > 0) {
+    const uint64_t a = bc[line], b = bc[before];
+    eq = (a & 255) == (b & 255) && text_equal(text, n_bytes, (int64_t)(a >> 8), (int64_t)(b >> 8), (uint32_t)(a & 255));
   }
-  pb = shfl_u64(b, below);
-  ph = shfl_u64(h, below);
-  if (lane == 0 && act && v > 0) {
-    const uint32_t line = kept[v - 1];
-    pb = bc[line];
-    ph = bch[line];
-  }
-  const uint32_t len = (uint32_t)(b & 255);
-  bool eq = act && v > 0 && h == ph && len == (uint32_t)(pb & 255);
-  for (uint32_t k = 0; ballot64(eq && k < len); k += 8) {
-    const uint64_t w = act && k < len ? load_u8x8(text, (int64_t)(b >> 8) + k, n_bytes) : 0;
-    uint64_t pw = shfl_u64(w, below);
-    if (eq && k < len) {
-      if (lane == 0) pw = load_u8x8(text, (int64_t)(pb >> 8) + k, n_bytes);
-      const uint64_t x = w ^ pw;
-      eq = (len - k < 8 ? first_bytes(x, len - k) : x) == 0;
-    }
-  }
-  if (act) run[v] = eq ? 0 : 1;
+  run[v] = eq ? 0 : 1;
 }
 
 // Groups of unsorted input: each record's barcode hash in a table of 2 n slots
@@ -1541,8 +1548,10 @@ int snapgpu_frag_index(const uint8_t* d_text, int64_t n_bytes, int64_t n_lines, 
   ParseOut po{at<uint32_t>(w, Lo.pos), at<uint32_t>(w, Lo.size), at<uint32_t>(w, Lo.cnt), at<uint8_t>(w, Lo.flags),
               at<uint64_t>(w, Lo.bc), at<uint64_t>(w, Lo.bch)};
   const int64_t lb = ceil_div(n_lines, kLineBlock);
+  const bool sorted = opt->sorted_by_barcode != 0;
+  uint8_t* same = sorted ? at<uint8_t>(w, Lo.wl) : nullptr;  // wl is written after the runs are known
   parse_kernel<<<(unsigned)lb, kThreads, 0, st>>>(d_text, n_bytes, line_start, n_lines, chroms, opt->shift_left,
-                                                  opt->shift_right, po, C, blk);
+                                                  opt->shift_right, po, C, blk, same);
   SG_LAUNCH_CHECK();
 
   // 3. compaction
@@ -1594,7 +1603,6 @@ int snapgpu_frag_index(const uint8_t* d_text, int64_t n_bytes, int64_t n_lines, 
   auto* gmito = at<unsigned long long>(w, Lo.gmito);
   auto* guniq = at<unsigned long long>(w, Lo.guniq);
   auto* gbad = at<unsigned int>(w, Lo.gbad);
-  const bool sorted = opt->sorted_by_barcode != 0;
   // key widths: positions below the genome length, values up to the largest size
   auto bits_of = [](uint64_t x) {
     int b = 1;
@@ -1610,7 +1618,7 @@ int snapgpu_frag_index(const uint8_t* d_text, int64_t n_bytes, int64_t n_lines, 
   SG_ARG(pos_bits + plan.vb <= 64, "position and value keys exceed 64 bits");
   int64_t G = 0;
   if (sorted) {
-    run_bound_kernel<<<grid(K), kThreads, 0, st>>>(d_text, n_bytes, kept, po.bc, po.bch, K, run);
+    run_bound_kernel<<<grid(K), kThreads, 0, st>>>(d_text, n_bytes, kept, po.bc, same, K, run);
     SG_LAUNCH_CHECK();
     rc = snapgpu_scan_inclusive_i64(run, K, sws, sws_bytes, stream);
     if (rc) return rc;

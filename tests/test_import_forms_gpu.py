@@ -90,3 +90,21 @@ def test_groups_of_unsorted_lines(torch_gpu, n, distinct):
     text = b"".join(b"chr1\t%d\t%d\tcell%d\t%d\n" % (s, s + 50, i, 1 + s % 3) for i, s in zip(ids, rng.integers(0, 900, n)))
     kw = dict(min_num_fragments=0, sorted_by_barcode=False)
     _check(_gpu(text, {"chr1": 1000}, **kw), import_text(text, {"chr1": 1000}, **kw))
+
+
+@pytest.mark.parametrize("width", [2, 8, 17, 100])
+@pytest.mark.parametrize("between", [b"", b"# note\n", b"chr1\t5\t5\tdropped\n", b"\n"])
+def test_runs_of_sorted_lines(torch_gpu, width, between):
+    """Runs that begin and end next to the parser's rounds of 256 lines and blocks of 4096,
+    barcodes that differ in their last character alone, and lines that are not kept between
+    records of one barcode."""
+    rng = np.random.default_rng(width)
+    n = 4096 + 700
+    cuts = np.zeros(n, int)
+    cuts[[1, 2, 63, 64, 65, 255, 256, 257, 511, 513, 1000, 4095, 4096, 4097, 4400]] = 1
+    run = np.cumsum(cuts)
+    names = [b"A" * (width - 1) + bytes([65 + r]) if r % 3 else b"A" * (width - 2) + bytes([97 + r]) for r in range(run[-1] + 1)]
+    text = b"".join((between if rng.random() < 0.02 else b"") + b"chr1\t%d\t%d\t%s\n" % (s, s + 30, names[r])
+                    for r, s in zip(run, rng.integers(0, 900, n)))
+    kw = dict(min_num_fragments=0)
+    _check(_gpu(text, {"chr1": 1000}, **kw), import_text(text, {"chr1": 1000}, **kw))
