@@ -90,6 +90,15 @@ def _degrees(X: DeviceCSR, w, torch):
     return 1.0 / op.dinv.cpu().numpy()
 
 
+def _scaled_rows(M, scale, torch):
+    """diag(scale) M with its rows on whole 128-byte lines: the sparse products gather
+    one row per entry, and a row of 30 doubles at a stride of 30 touches 2.75 lines
+    instead of 2 (192M entries, 250,000 rows: 7.1 ms, and 5.1 at a stride of 32)."""
+    n, k = M.shape
+    out = torch.empty((n, -(-k // 16) * 16), dtype=torch.float64, device=M.device)[:, :k]
+    return torch.mul(M, scale[:, None], out=out)
+
+
 def spectral_embedding_nystrom(X: DeviceCSR, n_components: int, sample_size: int,
                                weighted_by_degree: bool = False, chunk_size: int = 20000,
                                feature_weights=None, landmark_rows: np.ndarray | None = None,
@@ -129,18 +138,18 @@ def spectral_embedding_nystrom(X: DeviceCSR, n_components: int, sample_size: int
                                                 E.data_ptr(), k, st))
     # Z = seed~^T E = diag(w) X_seed^T diag(s_seed) E, on the landmark CSC; the
     # column scales are applied to the dense operand first (one gather per entry)
-    sE = (op.s[:, None] * E).contiguous()
+    sE = _scaled_rows(E, op.s, torch)
     Z = torch.empty((m, k), dtype=torch.float64, device=dev)
     _lib.check(L.snapgpu_csr_spmm_scaled_f64(op.colptr.data_ptr(), op.rowidx.data_ptr(), op.cval.data_ptr(),
-                                             m, w.data_ptr(), 0, sE.data_ptr(), k, k, Z.data_ptr(), k, st))
+                                             m, w.data_ptr(), 0, sE.data_ptr(), sE.stride(0), k, Z.data_ptr(), k, st))
     # q = sample~ Z = diag(s) X diag(w) Z for all cells
     s_all = torch.empty(n, dtype=torch.float64, device=dev)
     _lib.check(L.snapgpu_csr_row_inv_norm(X.indptr.data_ptr(), X.indices.data_ptr(), X.data.data_ptr(), n,
                                           w.data_ptr(), s_all.data_ptr(), st))
     Q = torch.empty((n, k), dtype=torch.float64, device=dev)
-    wZ = (w[:, None] * Z).contiguous()
+    wZ = _scaled_rows(Z, w, torch)
     _lib.check(L.snapgpu_csr_spmm_scaled_f64(X.indptr.data_ptr(), X.indices.data_ptr(), X.data.data_ptr(), n,
-                                             s_all.data_ptr(), 0, wZ.data_ptr(), k, k, Q.data_ptr(), k, st))
+                                             s_all.data_ptr(), 0, wZ.data_ptr(), wZ.stride(0), k, Q.data_ptr(), k, st))
     wsb = int(L.snapgpu_nystrom_normalize_workspace_bytes(n, k, chunk_size))
     ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
     _lib.check(L.snapgpu_nystrom_normalize(Q.data_ptr(), k, n, k, ev.data_ptr(), int(chunk_size), ws.data_ptr(),
