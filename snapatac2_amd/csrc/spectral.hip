@@ -1062,18 +1062,22 @@ static inline unsigned grid_for(int64_t work, int per_block, int64_t cap = 1 << 
 
 // --- C = A^T B over row chunks ------------------------------------------------
 // Up to 512 chunks of rows; each writes its ka x kb partial product, then the
-// partials are added in chunk order.
-static int64_t gemm_tn_chunks(int64_t n) {
-  return std::max<int64_t>(1, std::min<int64_t>(512, ceil_div(n, 4096)));
+// partials are added in chunk order. 4096 rows a chunk at a million rows; below
+// that down to 256, so that up to 256 blocks share the rows (3,001 rows, 16 x 16: 36 us
+// in one block, 7 in 12), as far as the partials fit the static scratch below.
+static int64_t gemm_tn_chunks(int64_t n, int32_t ka, int32_t kb) {
+  const int64_t least = std::max<int64_t>(1, std::min<int64_t>(512, ceil_div(n, 4096)));
+  const int64_t room = SNAPGPU_GEMM_TN_SCRATCH_BYTES / (8 * std::max<int64_t>(1, (int64_t)ka * kb));
+  return std::max(least, std::min({(int64_t)256, ceil_div(n, 256), room}));
 }
 
 static int64_t gemm_tn_partial_bytes(int64_t n, int32_t ka, int32_t kb) {
-  return gemm_tn_chunks(n) * (int64_t)ka * kb * 8;
+  return gemm_tn_chunks(n, ka, kb) * (int64_t)ka * kb * 8;
 }
 
 static int gemm_tn_launch(const double* d_A, int64_t lda, const double* d_B, int64_t ldb, int64_t n,
                           int32_t ka, int32_t kb, double* d_C, double* part, hipStream_t st) {
-  const int64_t chunks = gemm_tn_chunks(n);
+  const int64_t chunks = gemm_tn_chunks(n, ka, kb);
   const int64_t rpc = ceil_div(std::max<int64_t>(n, 1), chunks);
   // 16*TA columns of A per block: as few column groups as 128-wide ones need,
   // each as narrow as covers ka
