@@ -867,28 +867,67 @@ __global__ void group_key_kernel(const uint32_t* __restrict__ perm, const int64_
   key[j] = (uint64_t)run[perm[j]];
 }
 
-// Adds the QC sums of a wave's records (FragmentQCBuilder::update over the in-genome
-// records, qc.rs:442-449) to their groups, which are contiguous over the lanes: one
-// atomic per sum and group piece. `first`: the record before is of another group.
-__device__ __forceinline__ void add_group_sums(bool act, bool first, int64_t g, bool genome, bool is_mito, uint64_t tot,
-                                               unsigned long long* __restrict__ g_total,
-                                               unsigned long long* __restrict__ g_mito,
-                                               unsigned long long* __restrict__ g_uniq) {
-  const int lane = threadIdx.x & 63;
-  const uint64_t on = ballot64(act), heads = ballot64(act && (first || lane == 0));
-  const uint64_t mito = ballot64(act && genome && is_mito), uniq = ballot64(act && genome && !is_mito);
-  const uint64_t incl = wave_incl_scan_u64(act && genome ? tot : 0, lane);
-  const uint64_t upto = lanemask_lt(lane) | (1ull << lane);
-  const uint64_t own = heads & upto;
-  const int start = own ? 63 - __clzll((long long)own) : 0;
-  const uint64_t before = shfl_u64(incl, start > 0 ? start - 1 : 0);
-  const uint64_t piece = upto & ~lanemask_lt(start);
-  const bool tail = act && (lane == 63 || !((on & ~heads) >> (lane + 1) & 1));
-  if (!tail) return;
-  const uint64_t t = incl - (start > 0 ? before : 0), m = popc64(mito & piece), u = popc64(uniq & piece);
-  if (t) atomicAdd(&g_total[g], (unsigned long long)t);
-  if (m) atomicAdd(&g_mito[g], (unsigned long long)m);
-  if (u) atomicAdd(&g_uniq[g], (unsigned long long)u);
+// QC sums of the records of a wave (FragmentQCBuilder::update over the in-genome
+// records, qc.rs:442-449), which goes through kSumRounds * 64 consecutive records
+// and whose groups are contiguous: one atomic per sum and group. Atomics on one
+// address go one after the other; with one per 64 records they were most of the
+// time (55 million records, 8,000 groups: 545 us, 364 so; from the sorted keys of
+// 20.5 million records 250 us and 81).
+constexpr int kSumRounds = 8;
+constexpr int kSumBlockRecords = kThreads * kSumRounds;
+
+struct GroupSums {
+  unsigned long long *total, *mito, *uniq;
+  int64_t g = -1;  // the group whose records ended the last round; its sums (all lanes alike)
+  uint64_t t = 0;
+  uint32_t m = 0, u = 0;
+
+  __device__ __forceinline__ void add(int64_t g_, uint64_t t_, uint32_t m_, uint32_t u_) {
+    if (t_) atomicAdd(&total[g_], (unsigned long long)t_);
+    if (m_) atomicAdd(&mito[g_], (unsigned long long)m_);
+    if (u_) atomicAdd(&uniq[g_], (unsigned long long)u_);
+  }
+
+  // One record per lane (active lanes first). `first`: the record before is of another group.
+  __device__ __forceinline__ void round(bool act, bool first, int64_t gr, bool genome, bool is_mito, uint64_t cnt) {
+    const int lane = threadIdx.x & 63;
+    const uint64_t on = ballot64(act);
+    if (!on) return;
+    const uint64_t heads = ballot64(act && (first || lane == 0));
+    const uint64_t mitos = ballot64(act && genome && is_mito), uniqs = ballot64(act && genome && !is_mito);
+    const uint64_t incl = wave_incl_scan_u64(act && genome ? cnt : 0, lane);
+    const uint64_t upto = lanemask_lt(lane) | (1ull << lane);
+    const uint64_t own = heads & upto;
+    const int start = own ? 63 - __clzll((long long)own) : 0;
+    const uint64_t before = shfl_u64(incl, start > 0 ? start - 1 : 0);
+    const uint64_t piece = upto & ~lanemask_lt(start);
+    const int last = 63 - __clzll((long long)on);
+    uint64_t pt = incl - (start > 0 ? before : 0);
+    uint32_t pm = popc64(mitos & piece), pu = popc64(uniqs & piece);
+    const bool joins = (int64_t)shfl_u64((uint64_t)gr, 0) == g;
+    if (joins && start == 0) {
+      pt += t;
+      pm += m;
+      pu += u;
+    }
+    if (!joins && g >= 0 && lane == 0) add(g, t, m, u);
+    // pieces that end before the last active lane are complete
+    if (act && lane < last && (heads >> (lane + 1) & 1)) add(gr, pt, pm, pu);
+    g = (int64_t)shfl_u64((uint64_t)gr, last);
+    t = shfl_u64(pt, last);
+    m = __shfl(pm, last, 64);
+    u = __shfl(pu, last, 64);
+  }
+
+  __device__ __forceinline__ void finish() {
+    if (g >= 0 && (threadIdx.x & 63) == 0) add(g, t, m, u);
+  }
+};
+
+// First record of round r of this lane's wave.
+__device__ __forceinline__ int64_t sum_record(int r) {
+  return (int64_t)blockIdx.x * kSumBlockRecords + (int64_t)(threadIdx.x >> 6) * 64 * kSumRounds + r * 64 +
+         (threadIdx.x & 63);
 }
 
 // Sums, start slot and (sorted input) first line of each group, with the records in
@@ -899,25 +938,33 @@ __global__ void __launch_bounds__(kThreads) group_stats_kernel(
     const uint32_t* __restrict__ cnt_in, const int64_t* __restrict__ run, int64_t n, int64_t* __restrict__ gstart,
     uint32_t* __restrict__ gline, unsigned long long* __restrict__ g_total, unsigned long long* __restrict__ g_mito,
     unsigned long long* __restrict__ g_uniq) {
-  const int64_t j = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-  const bool act = j < n;
-  int64_t g = 0;
-  uint8_t f = 0;
-  uint64_t tot = 0;
-  bool first = false;
-  if (act) {
-    const int64_t v = perm ? perm[j] : j;
-    const uint32_t line = kept[v];
-    g = run[v] - 1;
-    f = flags[line];
-    tot = cnt_in[line];
-    first = j == 0 || run[perm ? perm[j - 1] : j - 1] - 1 != g;
-    if (first) {
-      gstart[g] = j;
-      if (!perm) gline[g] = line;
-    }
+  GroupSums sums{g_total, g_mito, g_uniq};
+  int64_t g[kSumRounds], prev[kSumRounds];
+  uint32_t line[kSumRounds], cnt[kSumRounds];
+  uint8_t f[kSumRounds];
+#pragma unroll
+  for (int r = 0; r < kSumRounds; ++r) {  // past the end: the last record, not used
+    const int64_t j = min(sum_record(r), n - 1), v = perm ? perm[j] : j;
+    line[r] = kept[v];
+    g[r] = run[v] - 1;
+    prev[r] = j > 0 ? run[perm ? perm[j - 1] : j - 1] - 1 : -1;
   }
-  add_group_sums(act, first, g, (f & F_GENOME) != 0, (f & F_MITO) != 0, tot, g_total, g_mito, g_uniq);
+#pragma unroll
+  for (int r = 0; r < kSumRounds; ++r) {
+    f[r] = flags[line[r]];
+    cnt[r] = cnt_in[line[r]];
+  }
+#pragma unroll
+  for (int r = 0; r < kSumRounds; ++r) {
+    const int64_t j = sum_record(r);
+    const bool act = j < n, first = act && prev[r] != g[r];
+    if (first) {
+      gstart[g[r]] = j;
+      if (!perm) gline[g[r]] = line[r];
+    }
+    sums.round(act, first, g[r], (f[r] & F_GENOME) != 0, (f[r] & F_MITO) != 0, cnt[r]);
+  }
+  sums.finish();
 }
 
 // The same from the sorted keys of unsorted input and the counts beside them.
@@ -927,20 +974,25 @@ __global__ void __launch_bounds__(kThreads) key_stats_kernel(const uint64_t* __r
                                                              unsigned long long* __restrict__ g_total,
                                                              unsigned long long* __restrict__ g_mito,
                                                              unsigned long long* __restrict__ g_uniq) {
-  const int64_t j = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-  const bool act = j < n;
-  int64_t g = 0;
-  uint64_t pv = 0, tot = 0;
-  bool first = false;
-  if (act) {
-    const uint64_t k = key[j];
-    g = (int64_t)key_group(k, plan);
-    pv = key_pv(k, plan);
-    tot = count[j];
-    first = j == 0 || (int64_t)key_group(key[j - 1], plan) != g;
-    if (first) gstart[g] = j;
+  GroupSums sums{g_total, g_mito, g_uniq};
+  uint64_t k[kSumRounds], before[kSumRounds];
+  uint32_t cnt[kSumRounds];
+#pragma unroll
+  for (int r = 0; r < kSumRounds; ++r) {  // past the end: the last record, not used
+    const int64_t j = min(sum_record(r), n - 1);
+    k[r] = key[j];
+    before[r] = key[j > 0 ? j - 1 : 0];
+    cnt[r] = count[j];
   }
-  add_group_sums(act, first, g, (pv >> (plan.vb + plan.mb)) < plan.total, (pv & 1) != 0, tot, g_total, g_mito, g_uniq);
+#pragma unroll
+  for (int r = 0; r < kSumRounds; ++r) {
+    const int64_t j = sum_record(r), g = (int64_t)key_group(k[r], plan);
+    const uint64_t pv = key_pv(k[r], plan);
+    const bool act = j < n, first = act && (j == 0 || (int64_t)key_group(before[r], plan) != g);
+    if (first) gstart[g] = j;
+    sums.round(act, first, g, (pv >> (plan.vb + plan.mb)) < plan.total, (pv & 1) != 0, cnt[r]);
+  }
+  sums.finish();
 }
 
 // Whether a whitelisted group holds a record that count_fragments cannot
@@ -1686,9 +1738,9 @@ int snapgpu_frag_index(const uint8_t* d_text, int64_t n_bytes, int64_t n_lines, 
   }
   SG_HIP(hipMemcpyAsync(at<SortPlan>(w, Lo.plan), &plan, sizeof(SortPlan), hipMemcpyHostToDevice, st));
   if (plan.one && !sorted)
-    key_stats_kernel<<<grid(K), kThreads, 0, st>>>(kb.Current(), vb.Current(), K, plan, gstart, gtot, gmito, guniq);
+    key_stats_kernel<<<grid(K, kSumBlockRecords), kThreads, 0, st>>>(kb.Current(), vb.Current(), K, plan, gstart, gtot, gmito, guniq);
   else
-    group_stats_kernel<<<grid(K), kThreads, 0, st>>>(sorted ? nullptr : perm, kept, po.flags, po.cnt, run, K, gstart,
+    group_stats_kernel<<<grid(K, kSumBlockRecords), kThreads, 0, st>>>(sorted ? nullptr : perm, kept, po.flags, po.cnt, run, K, gstart,
                                                      gline, gtot, gmito, guniq);
   SG_LAUNCH_CHECK();
   uint8_t* wl = at<uint8_t>(w, Lo.wl);
