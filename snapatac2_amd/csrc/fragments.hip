@@ -324,7 +324,7 @@ struct ParseOut {
   uint32_t* cnt;
   uint8_t* flags;
   uint64_t* bc;   // barcode offset << 8 | length
-  uint64_t* bch;  // hash of the barcode
+  uint64_t* bch;  // hash of the barcode (unsorted input, else null)
 };
 
 __device__ __forceinline__ uint64_t sat_add(uint64_t a, int64_t d) {
@@ -561,7 +561,7 @@ __device__ __forceinline__ uint64_t parse_line(const Text& t, const uint8_t* __r
             else pos = (uint32_t)(ce.base + coord);
           }
           bcw = ((uint64_t)f.bc_off << 8) | (f.bc_len > 255 ? 255u : f.bc_len);
-          if (err == 0) bch = hash_text(t, f.bc_off, f.bc_len);
+          if (err == 0 && out.bch) bch = hash_text(t, f.bc_off, f.bc_len);
         }
       }
     }
@@ -570,7 +570,7 @@ __device__ __forceinline__ uint64_t parse_line(const Text& t, const uint8_t* __r
     out.cnt[i] = count;
     out.flags[i] = err ? 0 : fl;
     out.bc[i] = bcw;
-    out.bch[i] = bch;
+    if (out.bch) out.bch[i] = bch;
     if (err) atomicMin(&cnt->err, ((unsigned long long)i << 8) | err);
     if (!err && (fl & F_KEEP)) {
       kept = bcw;
@@ -1008,24 +1008,27 @@ __global__ void bad_group_kernel(const unsigned int* __restrict__ g_bad, const u
 // Whitelist membership of each group's barcode (import.rs:74).
 __global__ void whitelist_kernel(const uint8_t* __restrict__ text, int64_t n_bytes,
                                  const uint32_t* __restrict__ gline,
-                                 const uint64_t* __restrict__ bc, const uint64_t* __restrict__ bch,
-                                 int64_t n_groups, const uint8_t* __restrict__ wl_table, uint8_t* __restrict__ wl) {
+                                 const uint64_t* __restrict__ bc, int64_t n_groups,
+                                 const uint8_t* __restrict__ wl_table, uint8_t* __restrict__ wl) {
   const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= n_groups) return;
   uint8_t w = 1;
   if (wl_table) {
-    const uint32_t line = gline[g];
-    const uint64_t b = bc[line];
-    w = table_find(wl_table, bch[line], FarText{text, n_bytes}, (int64_t)(b >> 8), (uint32_t)(b & 255)) >= 0 ? 1 : 0;
+    const uint64_t b = bc[gline[g]];
+    const FarText t{text, n_bytes};
+    w = table_find(wl_table, hash_text(t, (int64_t)(b >> 8), (uint32_t)(b & 255)), t, (int64_t)(b >> 8),
+                   (uint32_t)(b & 255)) >= 0 ? 1 : 0;
   }
   wl[g] = w;
 }
 
-__global__ void group_hash_kernel(const uint32_t* __restrict__ gline, const uint64_t* __restrict__ bch,
+__global__ void group_hash_kernel(const uint8_t* __restrict__ text, int64_t n_bytes,
+                                  const uint32_t* __restrict__ gline, const uint64_t* __restrict__ bc,
                                   int64_t n_groups, uint64_t* __restrict__ key, uint32_t* __restrict__ idx) {
   const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= n_groups) return;
-  key[g] = bch[gline[g]];
+  const uint64_t b = bc[gline[g]];
+  key[g] = hash_text(FarText{text, n_bytes}, (int64_t)(b >> 8), (uint32_t)(b & 255));
   idx[g] = (uint32_t)g;
 }
 
@@ -1598,7 +1601,7 @@ int snapgpu_frag_index(const uint8_t* d_text, int64_t n_bytes, int64_t n_lines, 
   c0.dup = ~0ull;
   SG_HIP(hipMemcpyAsync(C, &c0, sizeof(Counters), hipMemcpyHostToDevice, st));
   ParseOut po{at<uint32_t>(w, Lo.pos), at<uint32_t>(w, Lo.size), at<uint32_t>(w, Lo.cnt), at<uint8_t>(w, Lo.flags),
-              at<uint64_t>(w, Lo.bc), at<uint64_t>(w, Lo.bch)};
+              at<uint64_t>(w, Lo.bc), opt->sorted_by_barcode ? nullptr : at<uint64_t>(w, Lo.bch)};
   const int64_t lb = ceil_div(n_lines, kLineBlock);
   const bool sorted = opt->sorted_by_barcode != 0;
   uint8_t* same = sorted ? at<uint8_t>(w, Lo.wl) : nullptr;  // wl is written after the runs are known
@@ -1744,7 +1747,7 @@ int snapgpu_frag_index(const uint8_t* d_text, int64_t n_bytes, int64_t n_lines, 
                                                      gline, gtot, gmito, guniq);
   SG_LAUNCH_CHECK();
   uint8_t* wl = at<uint8_t>(w, Lo.wl);
-  whitelist_kernel<<<grid(G), kThreads, 0, st>>>(d_text, n_bytes, gline, po.bc, po.bch, G,
+  whitelist_kernel<<<grid(G), kThreads, 0, st>>>(d_text, n_bytes, gline, po.bc, G,
                                                  static_cast<const uint8_t*>(d_whitelist), wl);
   SG_LAUNCH_CHECK();
   uint32_t* ordA = at<uint32_t>(w, Lo.ordA);
@@ -1752,7 +1755,7 @@ int snapgpu_frag_index(const uint8_t* d_text, int64_t n_bytes, int64_t n_lines, 
   uint64_t* gkA = at<uint64_t>(w, Lo.gkA);
   uint64_t* gkB = at<uint64_t>(w, Lo.gkB);
   if (sorted && G > 1) {
-    group_hash_kernel<<<grid(G), kThreads, 0, st>>>(gline, po.bch, G, gkA, ordA);
+    group_hash_kernel<<<grid(G), kThreads, 0, st>>>(d_text, n_bytes, gline, po.bc, G, gkA, ordA);
     SG_LAUNCH_CHECK();
     hipcub::DoubleBuffer<uint64_t> gk(gkA, gkB);
     hipcub::DoubleBuffer<uint32_t> go(ordA, ordB);
