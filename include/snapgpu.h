@@ -615,6 +615,12 @@ int64_t snapgpu_frag_workspace_bytes(int64_t n_bytes, int64_t n_lines);
 int snapgpu_frag_index(const uint8_t* d_text, int64_t n_bytes, int64_t n_lines, const void* d_chroms,
                        const void* d_whitelist, const snapgpu_frag_options* opt, void* d_ws, int64_t ws_bytes,
                        snapgpu_frag_summary* h_summary, void* stream);
+/* The same with the workspace that snapgpu_frag_count_lines has just filled for this
+ * text (NULL: the lines are counted again). */
+int snapgpu_frag_index_counted(const uint8_t* d_text, int64_t n_bytes, int64_t n_lines, const void* d_count_ws,
+                               int64_t count_ws_bytes, const void* d_chroms, const void* d_whitelist,
+                               const snapgpu_frag_options* opt, void* d_ws, int64_t ws_bytes,
+                               snapgpu_frag_summary* h_sum, void* stream);
 /* d_cell_ptr[n_rows + 1], d_pos[nnz], d_val[nnz]; d_qc[3 n_rows] (optional):
  * per row n_fragment (unique), total count, mitochondrial; d_names[n_rows x
  * name_width] (optional): barcodes, zero padded. */

@@ -111,6 +111,7 @@ SIGNATURES: dict[str, tuple] = {
     "snapgpu_frag_count_lines": (C.c_int, [_p, _i64, _p, _i64, C.POINTER(_i64), _p]),
     "snapgpu_frag_workspace_bytes": (_i64, [_i64, _i64]),
     "snapgpu_frag_index": (C.c_int, [_p, _i64, _i64, _p, _p, _p, _p, _i64, _p, _p]),
+    "snapgpu_frag_index_counted": (C.c_int, [_p, _i64, _i64, _p, _i64, _p, _p, _p, _p, _i64, _p, _p]),
     "snapgpu_frag_fill": (C.c_int, [_p, _i64, _p, _i64, _p, _p, _p, _p, _p, _p, _i32, _p]),
     "snapgpu_csr_take_rows_workspace_bytes": (_i64, [_i64]),
     "snapgpu_csr_take_rows_count": (C.c_int, [_p, _i64, _p, _i64, _p, _p, _i64, C.POINTER(_i64), _p]),

@@ -279,9 +279,10 @@ __global__ void __launch_bounds__(kThreads) nl_count_kernel(const uint8_t* __res
 }
 
 // line_start[0] = 0 and line_start[k + 1] = (position of newline k) + 1.
-// blk_incl: inclusive scan of the per-block newline counts.
+// blk_incl: inclusive scan of the per-block newline counts; n_lines bounds the writes
+// (a text that has changed since it was counted).
 __global__ void __launch_bounds__(kThreads) nl_index_kernel(const uint8_t* __restrict__ text, int64_t n,
-                                                            const int64_t* __restrict__ blk_incl,
+                                                            const int64_t* __restrict__ blk_incl, int64_t n_lines,
                                                             int64_t* __restrict__ line_start) {
   __shared__ int64_t wsum[kThreads / 64];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -306,7 +307,7 @@ __global__ void __launch_bounds__(kThreads) nl_index_kernel(const uint8_t* __res
     while (m) {
       const int k = __ffs(m) - 1;
       m &= m - 1;
-      line_start[1 + o] = wi * 16 + k + 1;
+      if (o < n_lines) line_start[1 + o] = wi * 16 + k + 1;
       ++o;
     }
     base += total;
@@ -1554,7 +1555,17 @@ int64_t snapgpu_frag_workspace_bytes(int64_t n_bytes, int64_t n_lines) {
 int snapgpu_frag_index(const uint8_t* d_text, int64_t n_bytes, int64_t n_lines, const void* d_chroms,
                        const void* d_whitelist, const snapgpu_frag_options* opt, void* d_ws, int64_t ws_bytes,
                        snapgpu_frag_summary* h_sum, void* stream) {
+  return snapgpu_frag_index_counted(d_text, n_bytes, n_lines, nullptr, 0, d_chroms, d_whitelist, opt, d_ws, ws_bytes,
+                                    h_sum, stream);
+}
+
+int snapgpu_frag_index_counted(const uint8_t* d_text, int64_t n_bytes, int64_t n_lines, const void* d_count_ws,
+                               int64_t count_ws_bytes, const void* d_chroms, const void* d_whitelist,
+                               const snapgpu_frag_options* opt, void* d_ws, int64_t ws_bytes,
+                               snapgpu_frag_summary* h_sum, void* stream) {
   clear_error();
+  SG_ARG(d_count_ws == nullptr || count_ws_bytes >= snapgpu_frag_count_workspace_bytes(n_bytes),
+         "count workspace too small");
   SG_ARG(n_bytes >= 0 && n_lines >= 0 && opt != nullptr && h_sum != nullptr && d_chroms != nullptr,
          "bad arguments");
   SG_ARG(n_bytes == 0 || ((uintptr_t)d_text & 15) == 0, "text must be 16-byte aligned");
@@ -1577,18 +1588,23 @@ int snapgpu_frag_index(const uint8_t* d_text, int64_t n_bytes, int64_t n_lines, 
 
   // 1. line starts (the sentinel after a last line without '\n' is n_bytes + 1)
   const int64_t nb = ceil_div(n_bytes, kByteBlock);
-  nl_count_kernel<<<(unsigned)nb, kThreads, 0, st>>>(d_text, n_bytes, blk);
-  SG_LAUNCH_CHECK();
-  int rc = snapgpu_scan_inclusive_i64(blk, nb, sws, sws_bytes, stream);
-  if (rc) return rc;
+  int rc = SNAPGPU_OK;
+  const int64_t* nl = at<int64_t>(const_cast<void*>(d_count_ws), 0);  // the counts' scan
+  if (d_count_ws == nullptr) {
+    nl_count_kernel<<<(unsigned)nb, kThreads, 0, st>>>(d_text, n_bytes, blk);
+    SG_LAUNCH_CHECK();
+    rc = snapgpu_scan_inclusive_i64(blk, nb, sws, sws_bytes, stream);
+    if (rc) return rc;
+    nl = blk;
+  }
   // line_start holds n_lines + 1 entries: check n_lines before writing them
   int64_t n_nl = 0;
   uint8_t last = 0;
-  SG_HIP(hipMemcpyAsync(&n_nl, blk + nb - 1, 8, hipMemcpyDeviceToHost, st));
+  SG_HIP(hipMemcpyAsync(&n_nl, nl + nb - 1, 8, hipMemcpyDeviceToHost, st));
   SG_HIP(hipMemcpyAsync(&last, d_text + n_bytes - 1, 1, hipMemcpyDeviceToHost, st));
   SG_HIP(hipStreamSynchronize(st));
   SG_ARG(n_lines == n_nl + (last != '\n' ? 1 : 0), "n_lines does not match the text");
-  nl_index_kernel<<<(unsigned)nb, kThreads, 0, st>>>(d_text, n_bytes, blk, line_start);
+  nl_index_kernel<<<(unsigned)nb, kThreads, 0, st>>>(d_text, n_bytes, nl, n_lines, line_start);
   SG_LAUNCH_CHECK();
   const int64_t sentinel = n_bytes + 1;  // end of a last line without '\n'
   if (last != '\n') SG_HIP(hipMemcpyAsync(line_start + n_lines, &sentinel, 8, hipMemcpyHostToDevice, st));

@@ -92,15 +92,15 @@ def import_fragment_text(text, chrom_sizes: dict[str, int], *, min_num_fragments
     cws = torch.empty(L.snapgpu_frag_count_workspace_bytes(n_bytes), dtype=torch.uint8, device=dev)
     _lib.check(L.snapgpu_frag_count_lines(d_text.data_ptr(), n_bytes, cws.data_ptr(), cws.numel(),
                                           C.byref(n_lines), st))
-    del cws
     wsb = L.snapgpu_frag_workspace_bytes(n_bytes, n_lines.value)
     ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
     opt = _lib.FragOptions(int(shift_left), int(shift_right), max(int(min_num_fragments), 0),
                            1 if sorted_by_barcode else 0, 0)
     summ = _lib.FragSummary()
-    _lib.check(L.snapgpu_frag_index(d_text.data_ptr(), n_bytes, n_lines.value, d_chroms.data_ptr(),
-                                    None if d_wl is None else d_wl.data_ptr(), C.byref(opt),
-                                    ws.data_ptr(), wsb, C.byref(summ), st))
+    _lib.check(L.snapgpu_frag_index_counted(d_text.data_ptr(), n_bytes, n_lines.value, cws.data_ptr(), cws.numel(),
+                                            d_chroms.data_ptr(), None if d_wl is None else d_wl.data_ptr(),
+                                            C.byref(opt), ws.data_ptr(), wsb, C.byref(summ), st))
+    del cws
     R, nnz, width = summ.n_rows, summ.nnz, max(summ.name_width, 1)
     cell_ptr = torch.empty(R + 1, dtype=torch.int64, device=dev)
     pos = torch.empty(nnz, dtype=torch.int32, device=dev)
