@@ -5,7 +5,7 @@ X~ = rownorm(X diag(w)) and D = diag(X~ X~^T 1 - 1): the operator that
 snapatac2-python/src/embedding.rs:131-171 builds (with the weighting of
 embedding.rs:314-326) and that `spectral(feature_weights=...)` diagonalises
 (snapatac2/tools/_embedding.py:139,249). The reference has no derivative of it;
-the backward here is hand-written (csrc/spectral.hip, snapgpu_spectral_vjp_w):
+the backward here is hand-written (csrc/spectral.hip, snapgpu_spectral_vjp):
 
     dV = A(w) G                      (A is symmetric)
     dw = d<G, A(w) V>/dw             (explicit w^2, row norms and degrees)

@@ -108,3 +108,18 @@ def test_runs_of_sorted_lines(torch_gpu, width, between):
                     for r, s in zip(run, rng.integers(0, 900, n)))
     kw = dict(min_num_fragments=0)
     _check(_gpu(text, {"chr1": 1000}, **kw), import_text(text, {"chr1": 1000}, **kw))
+
+
+@pytest.mark.parametrize("last", [b"\n", b""])
+def test_lines_counted_again(torch_gpu, monkeypatch, last):
+    """The index that counts the lines by itself, and a line count that does not match."""
+    from snapatac2_amd import _lib
+    text = b"".join(b"chr1\t%d\t%d\tb%d\n" % (s, s + 9, s // 300) for s in range(1, 5000, 3))[:-1] + last
+    ref = import_text(text, {"chr1": 6000}, min_num_fragments=0)
+    L, off = _lib.lib(), [0]
+    monkeypatch.setattr(L, "snapgpu_frag_index_counted",
+                        lambda t, nb, nl, c, cb, *rest: L.snapgpu_frag_index(t, nb, nl + off[0], *rest))
+    _check(_gpu(text, {"chr1": 6000}, min_num_fragments=0), ref)
+    off[0] = -1
+    with pytest.raises(Exception, match="n_lines"):
+        _gpu(text, {"chr1": 6000}, min_num_fragments=0)
