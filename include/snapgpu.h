@@ -728,20 +728,22 @@ int64_t snapgpu_embed_workspace_bytes(int64_t n, int32_t kc);
 int snapgpu_embed_finish(const double* d_U, int64_t ldu, int64_t n, const int32_t* d_cols, int32_t kc,
                          const double* d_scale, double* d_out, void* d_ws, int64_t ws_bytes, void* stream);
 
-/* Host side of the peak matrix. snapgpu_region_parse: n items separated by '\n',
- * each "chrom:start-end" (GenomicRange::from_str, matrix.rs:113-124); *plain = 1 and
- * the distinct regions in first-occurrence order (chromosome id or -1, start, end,
+/* Regions of the peak matrix. snapgpu_region_parse (host only): n items separated by
+ * '\n', each "chrom:start-end" (GenomicRange::from_str, matrix.rs:113-124); *plain = 1
+ * and the distinct regions in first-occurrence order (chromosome id or -1, start, end,
  * index of their first item; arrays of n) when every item is printable ASCII without
  * blanks whose numbers have no sign or leading zero, *plain = 0 (outputs undefined)
  * otherwise. snapgpu_region_index: the arrays of snapgpu_peak_index for n regions
- * (those with chromosome -1 left out): by chromosome, start and index, with the running
- * maxima of the ends and the chromosomes' offsets h_off[n_chrom + 1]. */
+ * (those with chromosome -1 come last): by chromosome, start (none above max_start) and
+ * index, with the running maxima of the ends and the chromosomes' offsets
+ * d_off[n_chrom + 1]. */
 int snapgpu_region_parse(const char* h_text, int64_t n_bytes, int64_t n, const char* const* h_chroms,
                          int32_t n_chrom, int32_t* h_chrom, int64_t* h_start, int64_t* h_end, int64_t* h_first,
                          int64_t* n_distinct, int32_t* plain);
-int snapgpu_region_index(const int32_t* h_chrom, const int64_t* h_start, const int64_t* h_end, int64_t n,
-                         int32_t n_chrom, uint64_t* h_starts, uint64_t* h_ends, uint64_t* h_pmax, uint32_t* h_idx,
-                         int64_t* h_off);
+int64_t snapgpu_region_index_workspace_bytes(int64_t n);
+int snapgpu_region_index(const int32_t* d_chrom, const int64_t* d_start, const int64_t* d_end, int64_t n,
+                         int32_t n_chrom, int64_t max_start, uint64_t* d_starts, uint64_t* d_ends, uint64_t* d_pmax,
+                         uint32_t* d_idx, int64_t* d_off, void* d_ws, int64_t ws_bytes, void* stream);
 
 /* Gene level of the gene matrix (create_gene_matrix with id_type "gene",
  * feature_count/matrix.rs:173-273; GeneCount::get_values, counter.rs:270-283):

@@ -88,7 +88,8 @@ SIGNATURES: dict[str, tuple] = {
     "snapgpu_col_sums_f64": (C.c_int, [_p, _i64, _p, _p, _p]),
     "snapgpu_region_parse": (C.c_int, [C.c_char_p, _i64, _i64, C.POINTER(C.c_char_p), _i32, _p, _p, _p, _p,
                                        C.POINTER(_i64), C.POINTER(_i32)]),
-    "snapgpu_region_index": (C.c_int, [_p, _p, _p, _i64, _i32, _p, _p, _p, _p, _p]),
+    "snapgpu_region_index_workspace_bytes": (_i64, [_i64]),
+    "snapgpu_region_index": (C.c_int, [_p, _p, _p, _i64, _i32, _i64, _p, _p, _p, _p, _p, _p, _i64, _p]),
     "snapgpu_embed_workspace_bytes": (_i64, [_i64, _i32]),
     "snapgpu_embed_finish": (C.c_int, [_p, _i64, _i64, _p, _i32, _p, _p, _p, _i64, _p]),
     "snapgpu_spectral_vjp_products_workspace_bytes": (_i64, [_i64, _i64, _i32]),

@@ -88,19 +88,23 @@ def parse_region_arrays(peaks, chroms) -> tuple[list[str], RegionArrays]:
     return items, RegionArrays(chrom[:k], start[:k], end[:k])
 
 
-def region_index(r: RegionArrays, n_chrom: int):
-    """(starts, ends, running maxima of the ends, region, chromosome offsets): the
-    regions of each chromosome by start and index (snapgpu_peak_index)."""
+def region_index(r: RegionArrays, n_chrom: int, torch):
+    """Device tensors (starts, ends, running maxima of the ends, region, chromosome
+    offsets): the regions of each chromosome by start and index (snapgpu_region_index)."""
+    L = _lib.lib()
+    dev = torch.device("cuda")
     n = len(r)
-    size = max(n, 1)
-    starts, ends, pmax = (np.zeros(size, dtype=np.uint64) for _ in range(3))
-    index = np.zeros(size, dtype=np.uint32)
-    off = np.zeros(n_chrom + 1, dtype=np.int64)
-    chrom, start, end = (np.ascontiguousarray(a, dtype=t) for a, t in
+    chrom, start, end = (torch.from_numpy(np.ascontiguousarray(a, dtype=t)).to(dev) for a, t in
                          ((r.chrom, np.int32), (r.start, np.int64), (r.end, np.int64)))
-    _lib.check(_lib.lib().snapgpu_region_index(
-        chrom.ctypes.data, start.ctypes.data, end.ctypes.data, n, n_chrom, starts.ctypes.data, ends.ctypes.data,
-        pmax.ctypes.data, index.ctypes.data, off.ctypes.data))
+    starts, ends, pmax = (torch.empty(max(n, 1), dtype=torch.int64, device=dev) for _ in range(3))
+    index = torch.empty(max(n, 1), dtype=torch.int32, device=dev)
+    off = torch.empty(n_chrom + 1, dtype=torch.int64, device=dev)
+    wsb = int(L.snapgpu_region_index_workspace_bytes(n))
+    ws = torch.empty(max(wsb, 1), dtype=torch.uint8, device=dev)
+    _lib.check(L.snapgpu_region_index(
+        chrom.data_ptr(), start.data_ptr(), end.data_ptr(), n, n_chrom, int(np.max(r.start, initial=0)),
+        starts.data_ptr(), ends.data_ptr(), pmax.data_ptr(), index.data_ptr(), off.data_ptr(), ws.data_ptr(), wsb,
+        _lib.stream_ptr()))
     return starts, ends, pmax, index, off
 
 
@@ -112,10 +116,8 @@ class PeakIndex:
         dev = torch.device("cuda")
         chroms = list(chrom_sizes)
         r = regs if isinstance(regs, RegionArrays) else RegionArrays.of(regs, chroms)
-        starts, ends, pmax, index, off = region_index(r, len(chroms))
         base = np.concatenate([[0], np.cumsum([int(chrom_sizes[c]) for c in chroms])]).astype(np.uint64)
-        t = lambda a: torch.from_numpy(np.ascontiguousarray(a).view(np.int64 if a.dtype.itemsize == 8 else np.int32)).to(dev)
-        self._keep = [t(a) for a in (starts, ends, pmax, index, off, base)]
+        self._keep = [*region_index(r, len(chroms), torch), torch.from_numpy(base.view(np.int64)).to(dev)]
         self.c = _lib.PeakIndex(*[x.data_ptr() for x in self._keep], len(chroms), len(r))
 
 

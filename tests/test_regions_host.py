@@ -113,11 +113,11 @@ def test_bin_index_ranges_equal_the_names():
     assert list(bi.to_numpy()) == ["chr1:0-500", "chr1:500-1000", "chr1:1000-1234", "chr10:0-500", "chr2:0-1"]
 
 
-# --- the native parse and index of the peak matrix ---------------------------
+# --- the native parse of the peak matrix ---------------------------
 
 import numpy as np  # noqa: E402
 
-from snapatac2_amd.pp._peaks import RegionArrays, parse_region_arrays, region_index  # noqa: E402
+from snapatac2_amd.pp._peaks import RegionArrays, parse_region_arrays  # noqa: E402
 
 CHROMS = ["chr1", "chr2", "HLA:A", "é", "chr1\0x"]
 PLAIN = ["chr2:1-2", "chr1:5-10", "chr1:0-0", "chr1:5-10", "HLA:A:7-9", ":3-4", "chrU:5-10", "chr1:5-11", "chr1:50-1",
@@ -144,20 +144,3 @@ def test_region_arrays_refuse_what_the_parse_refuses(bad):
     for items in ([bad], PLAIN + [bad], [bad] + PLAIN):
         with pytest.raises(_lib.PanicException):
             parse_region_arrays(items, CHROMS)
-
-
-@pytest.mark.parametrize("n", [0, 1, 2, 300])
-def test_region_index_equals_a_stable_sort(n):
-    rng = np.random.default_rng(n)
-    chrom = rng.integers(-1, 4, n).astype(np.int32)  # -1: outside the genome; chromosome 4 of 5 stays empty
-    start, end = rng.integers(0, 40, n), rng.integers(0, 90, n)
-    starts, ends, pmax, index, off = region_index(RegionArrays(chrom, start, end), 5)
-    order = np.lexsort((np.arange(n), start, chrom))
-    order = order[chrom[order] >= 0]
-    k = len(order)
-    assert np.array_equal(index[:k], order) and np.array_equal(starts[:k], start[order])
-    assert np.array_equal(ends[:k], end[order])
-    assert np.array_equal(off, np.searchsorted(chrom[order], np.arange(6)))
-    for c in range(5):
-        a, b = off[c], off[c + 1]
-        assert np.array_equal(pmax[a:b], np.maximum.accumulate(end[order][a:b]))
