@@ -592,7 +592,7 @@ __device__ __forceinline__ uint64_t parse_line(const Text& t, const uint8_t* __r
 // The text of a round's 256 lines is read once, in order, into LDS (kStage bytes; 16
 // below it and kStagePad above are read past a line's ends and masked away): a lane
 // reads its line in some thirty pieces, and from global memory those went to L2 again
-// and again (2.94 ms for 55 million lines of 41 characters that way, 1.99 ms staged;
+// and again (2.94 ms for 55 million lines of 41 characters that way, 1.93 ms staged;
 // 4.13 ms one character after the other, 0.9 ms the copy of the bytes alone). Rounds of longer lines read
 // the text where it lies, one character after the other.
 constexpr int kStage = 16384, kStagePad = 96;
@@ -1721,9 +1721,9 @@ int snapgpu_frag_index_counted(const uint8_t* d_text, int64_t n_bytes, int64_t n
   h_sum->n_groups = G;
 
   // 5. sort, and 6. group sums. One sort where the key's bits suffice: 55 million
-  // records of 8,000 barcodes take 2.3 ms of sorting and 1.2 ms of key, sums and fill
+  // records of 8,000 barcodes take 2.3 ms of sorting and 0.95 ms of key, sums and fill
   // kernels; two sorts through a permutation and its gathers 3.8 and 2.4 ms. (20.5
-  // million unsorted records: 1.4 and 0.5 ms; with a sort of 64-bit hashes 2.6 and 5.9.)
+  // million unsorted records: 1.4 and 0.3 ms; with a sort of 64-bit hashes 2.6 and 5.9.)
   const int gbits = G > 1 ? bits_of((uint64_t)(G - 1)) : 0;
   plan.mb = sorted ? 0 : 1;
   plan.pv = pos_bits + plan.vb + plan.mb;
