@@ -328,7 +328,8 @@ __global__ void __launch_bounds__(kThreads) product_kernel(
     // same window. A quad's chunk is nine entries on average at 891 million
     // entries in 778 blocks x 489 windows, so what is taken at once is small: per
     // application 11.93 ms with 24 loaded ahead and 8 at a time, 11.71 with 16 and
-    // 8, 11.28 with 16 and 4, 11.39 with 8 and 4.
+    // 8, 11.28 with 16 and 4, 11.39 with 8 and 4; 1.9 billion in 982 blocks (sixteen
+    // a chunk) 22.14 with 24 and 8, 21.56 with 24 and 4, 21.84 with 16 and 4.
     constexpr int kPre = SNAPGPU_WINDOW_PRE, kStep = SNAPGPU_WINDOW_STEP;
     const int64_t bq0 = blk * nw;
     int64_t bs = bstart[bq0 + w0];
