@@ -1075,6 +1075,17 @@ static int64_t gemm_tn_partial_bytes(int64_t n, int32_t ka, int32_t kb) {
   return gemm_tn_chunks(n, ka, kb) * (int64_t)ka * kb * 8;
 }
 
+// Bytes that hold the partials of every product of these rows with at most ka and kb
+// columns. A narrower product may take more chunks, and more bytes with them, but no
+// more than the scratch where it goes past `least`. A solver sizes one workspace for
+// its widest product.
+static int64_t gemm_tn_bytes_up_to(int64_t n, int32_t ka, int32_t kb) {
+  const int64_t one = 8 * (int64_t)ka * kb;
+  const int64_t least = std::max<int64_t>(1, std::min<int64_t>(512, ceil_div(n, 4096)));
+  return std::max(least * one, std::min(std::min<int64_t>(256, ceil_div(n, 256)) * one,
+                                        (int64_t)SNAPGPU_GEMM_TN_SCRATCH_BYTES));
+}
+
 static int gemm_tn_launch(const double* d_A, int64_t lda, const double* d_B, int64_t ldb, int64_t n,
                           int32_t ka, int32_t kb, double* d_C, double* part, hipStream_t st) {
   const int64_t chunks = gemm_tn_chunks(n, ka, kb);
@@ -1471,7 +1482,7 @@ int snapgpu_spectral_vjp_w_mixed(const snapgpu_window_layout* csr_windows, const
 }
 
 int64_t snapgpu_gemm_tn_workspace_bytes(int64_t n, int32_t ka, int32_t kb) {
-  return gemm_tn_partial_bytes(n, ka, kb) + 256;
+  return gemm_tn_bytes_up_to(n, ka, kb) + 256;
 }
 
 // C[ka x kb] = A[n x ka]^T B[n x kb] (row-major, leading dims lda/ldb).
@@ -1481,7 +1492,7 @@ int snapgpu_gemm_tn_f64(const double* d_A, int64_t lda, const double* d_B, int64
   clear_error();
   SG_ARG(ka >= 1 && kb >= 1 && kb <= 32, "need 1 <= kb <= 32");
   SG_ARG(n >= 0 && lda >= ka && ldb >= kb, "need n >= 0, lda >= ka, ldb >= kb");
-  SG_ARG(ws_bytes >= snapgpu_gemm_tn_workspace_bytes(n, ka, kb), "workspace too small");
+  SG_ARG(ws_bytes >= gemm_tn_partial_bytes(n, ka, kb) + 256, "workspace too small");
   return gemm_tn_launch(d_A, lda, d_B, ldb, n, ka, kb, d_C, (double*)d_ws, as_stream(stream));
 }
 

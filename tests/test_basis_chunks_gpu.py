@@ -24,3 +24,22 @@ def test_row_chunks(torch_gpu, n, ka, kb):
     bound = 1e-13 * (A.abs().T @ B.abs())
     assert bool(((C - A.T @ B).abs() <= bound).all())
     assert torch.equal(C, D)
+
+
+def test_one_workspace_for_narrower_products(torch_gpu):
+    """The block Lanczos solver's use: a workspace of the widest basis, and a narrower product
+    that takes more row chunks (70,000 rows: 125 at 1041 x 32, 256 at 1024 x 16)."""
+    torch = torch_gpu
+    L = _lib.lib()
+    n = 70_000
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    A = torch.randn((n, 1041), dtype=torch.float64, device="cuda", generator=gen)
+    wsb = int(L.snapgpu_gemm_tn_workspace_bytes(n, 1041, 32))
+    ws = torch.empty(wsb, dtype=torch.uint8, device="cuda")
+    for ka, kb in ((1024, 16), (1041, 32), (17, 1)):
+        B = torch.randn((n, kb), dtype=torch.float64, device="cuda", generator=gen)
+        C = torch.empty((ka, kb), dtype=torch.float64, device="cuda")
+        _lib.check(L.snapgpu_gemm_tn_f64(A.data_ptr(), 1041, B.data_ptr(), kb, n, ka, kb, C.data_ptr(), ws.data_ptr(),
+                                         wsb, _lib.stream_ptr()))
+        bound = 1e-13 * (A[:, :ka].abs().T @ B.abs())
+        assert bool(((C - A[:, :ka].T @ B).abs() <= bound).all()), (ka, kb)
