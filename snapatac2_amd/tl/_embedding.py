@@ -12,6 +12,7 @@ from typing import Literal
 import numpy as np
 
 from .. import _lib
+from .._device import to_host
 from ._lanczos import eigsh_lm
 from ._operator import SpectralOperator, _to_device_csr, select_columns
 
@@ -49,11 +50,7 @@ def _finished(U, cols, scale=None) -> np.ndarray:
     ws = torch.empty(ws_b, dtype=torch.uint8, device=U.device)
     _lib.check(L.snapgpu_embed_finish(U.data_ptr(), U.stride(0), n, d_cols.data_ptr(), kc, _lib.ptr(d_scale),
                                       out.data_ptr(), ws.data_ptr(), ws_b, _lib.stream_ptr()))
-    # page-locked (the returned array keeps it alive): one DMA
-    host = torch.empty((n, kc), dtype=torch.float64, pin_memory=True)
-    host.copy_(out, non_blocking=True)
-    torch.cuda.current_stream().synchronize()
-    return host.numpy()
+    return to_host(out)
 
 
 def _eigenpairs(adata, features, n_components: int, random_state: int, feature_weights):
