@@ -16,6 +16,7 @@ def test_to_host(torch_gpu, monkeypatch, shape, dtype):
     torch = torch_gpu
     from snapatac2_amd import _device
     monkeypatch.setattr(_device, "_STAGE_BYTES", 2048)  # 256 doubles at a time
+    monkeypatch.setattr(_device, "_THREADED_BYTES", 1024)  # whole blocks by torch, most remainders by numpy
     a = np.random.default_rng(1).integers(-9, 9, shape).astype(dtype)
     got = _device.to_host(torch.from_numpy(a).cuda())
     assert got.dtype == a.dtype and got.shape == a.shape and np.array_equal(got, a)
