@@ -551,19 +551,25 @@ static int launch(const Params& p, hipStream_t st) {
 
 // ---------------------------------------------------------------------------
 // The segment kernel (level 0): a cell's fragments in segments of kSeg = 256,
-// four per lane, one wave each, the segments of a cell independent of each
-// other. Segment s owns the bins [B_s, B_{s+1}), B_s being the lower bound of
-// the bins from its first fragment on (B_0 = 0): it drops its own events at or
-// past B_{s+1} and looks back for the earlier fragments that reach B_s, which
-// begin at most kSpan bins before it. Start bins ascend, so the distinct start
-// bins U[1..G] of a segment come from a compare and a prefix sum, and a further
-// event (a second insertion, a covered bin) either meets one of them a few
-// places on or falls into a gap between two: each gap keeps a 32-bit mask of its
-// extra bins, so the row's order never has to be sorted. Entry 0 stands for the
-// gap from B_s to the first start bin. The number of entries is G plus the bits
-// of all masks; an event's rank is its gap's prefix plus the bits below it. The
-// fill pass adds the events into counts by rank in LDS (kRank at a time) and
-// writes them coalesced.
+// four per lane, one wave each. Segment s owns the bins [B_s, B_{s+1}), B_s being
+// the lower bound of the bins from its first fragment on (B_0 = 0); what its
+// fragments count in later bins is carried. A fragment begins at or below B_{s+1}
+// and covers at most kSpan bins past its first, so the carry is kCarry = 32 counts,
+// of the bins from B_{s+1} on, one per lane: each segment adds its own past events
+// to what of its carry lies at or past B_{s+1}. (Waves that share a cell put
+// their past events into LDS and each sums those before it.) The work is linear in
+// the fragments however they crowd: with a look back over the fragments within reach
+// of B_s instead, the matrix of 8,200 cells with 2,000 fragments over the genome and
+// 5,000 on 16 kb took 5.5 ms, 1.0 so (the tile kernel 1.9).
+//
+// Start bins ascend, so the distinct start bins U[1..G] of a segment come from a
+// compare and a prefix sum, and a further event (a second insertion, a covered bin,
+// a carried count) either meets one of them a few places on or falls into a gap
+// between two: each gap keeps a 32-bit mask of its extra bins, so the row's order
+// never has to be sorted. Entry 0 stands for the gap from B_s to the first start
+// bin. The number of entries is G plus the bits of all masks; an event's rank is
+// its gap's prefix plus the bits below it. The fill pass adds the events into
+// counts by rank in LDS (kRank at a time) and writes them coalesced.
 //
 // A fragment that covers more than kSpan bins does not fit a mask: the launch is
 // then repeated by the tile kernel above, which also takes bins so small that
@@ -576,6 +582,7 @@ static int launch(const Params& p, hipStream_t st) {
 constexpr int kSeg = 256;
 constexpr int kRank = 512;
 constexpr uint32_t kSpan = 31;      // b2 - b1 at most
+constexpr uint32_t kCarry = kSpan + 1;  // bins of the carry
 constexpr uint32_t kMinSegBin = 64;  // 32 bins of 64 bases: fragments of up to 2 kb
 constexpr int32_t kSegChroms = 1024;  // chromosomes at most: 16 waves' scratch and the table share LDS
 constexpr int64_t kSegCells16 = 1024, kSegCells4 = 8192;  // below: 16 and 4 waves per cell
@@ -587,6 +594,7 @@ struct alignas(4) Quad {
 template <bool FILL>
 struct SegLds {
   uint2 um[kSeg + 2];  // x: start bin U[g], y: mask of the extra bins in the gap after it
+  uint32_t past[2][kCarry];  // events at the bins from Bn on (two: one is read while the next is filled)
   uint32_t base[FILL ? kSeg + 2 : 1];  // rank of U[g] (entry 0: one below the gap's first)
   uint32_t cnt[FILL ? kRank : 1];
   uint32_t bin[FILL ? kRank : 1];
@@ -707,9 +715,10 @@ __device__ __forceinline__ void seg_load(const Params& p, int64_t a, int64_t f0,
 // when it differs), SNAPGPU_FRAGMENT (every covered bin) or SNAPGPU_SINGLE.
 // WAVES waves share one cell and take its segments in turn.
 template <int STRATEGY, int WAVES, bool FILL, typename IdxT>
-__device__ __forceinline__ void seg_cell(const Params& p, const ChromRec* tab, SegLds<FILL>* L, uint32_t* totals,
-                                         int64_t cell, int wave, int lane) {
+__device__ __forceinline__ void seg_cell(const Params& p, const ChromRec* tab, SegLds<FILL>* lds, uint32_t* totals,
+                                         uint32_t* stops, int64_t cell, int wave, int lane) {
   constexpr bool PAIRED = STRATEGY != SNAPGPU_SINGLE;
+  SegLds<FILL>* L = lds + wave;
   const int64_t f0 = (int64_t)p.cell_ptr[cell], f1 = (int64_t)p.cell_ptr[cell + 1];
   const int64_t f_all = (int64_t)p.cell_ptr[p.n_cells];
   const uint32_t genome = (uint32_t)tab[p.n_chrom].start;
@@ -718,6 +727,7 @@ __device__ __forceinline__ void seg_cell(const Params& p, const ChromRec* tab, S
   const int64_t out_end = FILL ? p.indptr[cell + 1] : 0;
   Chrom c{1, 0, 0, 0, 0}, cb{1, 0, 0, 0, 0};  // empty: the first position enters one
   uint32_t entries = 0;  // counting: this lane's share of the row's entries
+  uint32_t carry = 0;    // lane i < kCarry: events of the fragments before this round at its first bin + i
   bool overflow = false;
   SegLoad nxt;
   seg_load<PAIRED>(p, f0 + (int64_t)kSeg * wave, f0, f1, f_all, lane, nxt);
@@ -729,8 +739,9 @@ __device__ __forceinline__ void seg_cell(const Params& p, const ChromRec* tab, S
     uint32_t total = 0;
     uint32_t b1[4], b2[4], g[4], gs[4];
     bool k[4] = {false, false, false, false};
-    uint32_t B = 0, Bn = 0;
-    bool back = false;  // some earlier fragment may reach B
+    uint32_t B = kInf, Bn = kInf;
+    uint32_t top = 0;        // largest start bin of this lane that the segment owns, plus one
+    uint32_t own_carry = 0;  // lane i < kCarry: events of the fragments before the segment at B + i
     const int nf = (int)min<int64_t>(max<int64_t>(f1 - a, 0), kSeg);
     // an event at bin v: the gap it lies in, from entry `from` on
     uint32_t G = 0;
@@ -744,29 +755,8 @@ __device__ __forceinline__ void seg_cell(const Params& p, const ChromRec* tab, S
       if (d != 0 && d <= 32) atomicOr(&L->um[e].y, 1u << (d - 1));
       return e;
     };
-    // the events of the fragments before the segment that lie in [B, Bn)
-    const auto look_back = [&](auto&& f) {
-      Chrom cl = cb;
-      for (int64_t j1 = a; j1 > f0; j1 -= 64) {
-        const int64_t j = j1 - 64 + lane;
-        const uint32_t ps = p.pos[max(j, f0)];
-        const bool near = j >= f0 && (uint64_t)ps + 32ull * p.bin_size > s.first;
-        if (ballot64(near) == 0) break;
-        if (near) {
-          uint32_t x1, x2;
-          if (seg_decode<false>(p, tab, genome, inv, PAIRED, ps, PAIRED ? p.len[j] : 1u, cell, cl, x1, x2) &&
-              x2 - x1 <= kSpan) {
-            if (x1 >= B && x1 < Bn) f(x1);
-            if (STRATEGY == SNAPGPU_FRAGMENT) {
-              for (uint32_t v = x1 + 1; v <= x2; ++v)
-                if (v >= B && v < Bn) f(v);
-            } else if (PAIRED && (STRATEGY == SNAPGPU_INSERTION || x2 != x1)) {
-              if (x2 >= B && x2 < Bn) f(x2);
-            }
-          }
-        }
-      }
-    };
+    uint32_t* past = L->past[round & 1];  // filled if `reaches`
+    bool reaches = false;
     if (nf > 0) {
       // positions must ascend along the row: the order of the bins relies on it
       uint32_t prev = dpp_shr1(s.pos[3], s.before);
@@ -783,7 +773,6 @@ __device__ __forceinline__ void seg_cell(const Params& p, const ChromRec* tab, S
         if (lane == 0) report(p, kErrUnsorted, cell, 0);
         Bn = B = 0;  // owns nothing
       }
-      uint32_t top = 0;  // largest start bin of this lane, plus one
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         b1[r] = b2[r] = kInf;
@@ -793,10 +782,74 @@ __device__ __forceinline__ void seg_cell(const Params& p, const ChromRec* tab, S
           overflow = true;
           k[r] = false;
         }
+        if (!k[r]) b1[r] = b2[r] = 0;
+      }
+      // what lies past the segment's bins
+      bool reach = false;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) reach |= k[r] && b2[r] >= Bn;
+      reaches = ballot64(reach) != 0;
+      if (reaches) {
+        if (lane < (int)kCarry) past[lane] = 0u;
+        wave_sync();
+        const auto leave = [&](uint32_t v) {
+          if (v >= Bn && v - Bn < kCarry) atomicAdd(&past[v - Bn], 1u);
+        };
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if (!k[r] || b2[r] < Bn) continue;
+          if (STRATEGY == SNAPGPU_FRAGMENT) {
+            for (uint32_t v = max(b1[r], Bn); v <= b2[r]; ++v) leave(v);
+          } else {
+            leave(b1[r]);
+            if (PAIRED && (STRATEGY == SNAPGPU_INSERTION || b2[r] != b1[r])) leave(b2[r]);
+          }
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
         k[r] = k[r] && b1[r] < Bn && b1[r] >= B;
         if (k[r]) top = max(top, b1[r] + 1);
       }
-      back = a > f0 && Bn > B && (uint64_t)s.before + 32ull * p.bin_size > s.first;
+    }
+    // The carry into this segment and into the next round's first one. A lane's bin is
+    // x; what was counted there lies in the round's carry (from its first bin on) and
+    // in the past events of the segments before.
+    if (WAVES > 1) {
+      uint32_t* stop = stops + (round & 1) * (2 * WAVES + 1);  // B, then each wave's Bn, then `reaches`
+      if (lane == 0) {
+        stop[wave + 1] = Bn;
+        stop[WAVES + 1 + wave] = reaches ? 1u : 0u;
+        if (wave == 0) stop[0] = B;
+      }
+      __syncthreads();
+      // lane w: where wave w stopped, and whether it left anything there
+      const uint32_t stopped = stop[1 + (lane & (WAVES - 1))];
+      const bool left = lane < WAVES && stop[WAVES + 1 + (lane & (WAVES - 1))] != 0;
+      const uint32_t first = stop[0];
+      const uint32_t round_carry = carry;
+      const auto before = [&](uint32_t from, int waves) {  // at bin from + lane, by the round's first `waves`
+        const uint32_t d0 = from - first + lane;
+        uint32_t n = (uint32_t)__shfl((int)round_carry, (int)(d0 & 63), 64);
+        if (d0 >= kCarry) n = 0;
+        for (uint64_t m = ballot64(left && lane < waves && from - stopped < kCarry); m != 0; m &= m - 1) {
+          const int w = lowbit64(m);
+          const uint32_t d = from - (uint32_t)__builtin_amdgcn_readlane((int)stopped, w) + lane;
+          if (d < kCarry) n += lds[w].past[round & 1][d];
+        }
+        return lane < (int)kCarry ? n : 0u;
+      };
+      own_carry = before(stop[wave], wave);
+      carry = before(stop[WAVES], WAVES);
+    } else {
+      wave_sync();
+      own_carry = carry;
+      const uint32_t d = Bn - B + lane;
+      const uint32_t c0 = (uint32_t)__shfl((int)carry, (int)(d & 63), 64);
+      carry = lane < (int)kCarry ? (d < kCarry ? c0 : 0u) + (reaches ? past[lane] : 0u) : 0u;
+    }
+    if (nf > 0) {
+      const bool carried = own_carry != 0 && B + lane < Bn;  // lanes past the carry hold 0
       // distinct start bins, in order
       uint32_t seen = dpp_shr1(dpp_scan(top, [](uint32_t x, uint32_t y) { return max(x, y); }), 0u);
       bool fresh[4];
@@ -830,7 +883,7 @@ __device__ __forceinline__ void seg_cell(const Params& p, const ChromRec* tab, S
           if (k[r] && b2[r] != b1[r] && b2[r] < Bn) gs[r] = note(b2[r], g[r]);
         }
       }
-      if (back) look_back([&](uint32_t v) { note(v, 0); });
+      if (carried) note(B + lane, 0);
       wave_sync();
       uint32_t own = lane == 0 ? __popc(L->um[0].y) : 0u;
       uint32_t extra[4];
@@ -876,29 +929,29 @@ __device__ __forceinline__ void seg_cell(const Params& p, const ChromRec* tab, S
         const uint32_t n = min(total - r0, (uint32_t)kRank);
         for (uint32_t i = lane; i < n; i += 64) L->cnt[i] = 0u;
         wave_sync();
-        const auto add = [&](uint32_t v, uint32_t e) {  // an event at bin v, in the gap of entry e
+        const auto add = [&](uint32_t v, uint32_t e, uint32_t times) {  // events at bin v, in the gap of entry e
           const uint2 u = L->um[e];
           const uint32_t d = v - u.x;
           const uint32_t r = L->base[e] + (d == 0 ? 0u : __popc(u.y & ((2u << (d - 1)) - 1u))) - r0;
           if (r < n) {
             L->bin[r] = v;
-            atomicAdd(&L->cnt[r], 1u);
+            atomicAdd(&L->cnt[r], times);
           }
         };
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           if (!k[r]) continue;
-          add(b1[r], g[r]);
+          add(b1[r], g[r], 1u);
           if (STRATEGY == SNAPGPU_FRAGMENT) {
             for (uint32_t v = b1[r] + 1, e = g[r]; v <= b2[r] && v < Bn; ++v) {
               e = gap(v, e);
-              add(v, e);
+              add(v, e, 1u);
             }
           } else if (PAIRED && (STRATEGY == SNAPGPU_INSERTION || b2[r] != b1[r])) {
-            if (b2[r] < Bn) add(b2[r], gs[r]);
+            if (b2[r] < Bn) add(b2[r], gs[r], 1u);
           }
         }
-        if (back) look_back([&](uint32_t v) { add(v, gap(v, 0)); });
+        if (own_carry != 0 && B + lane < Bn) add(B + lane, gap(B + lane, 0), own_carry);
         wave_sync();
         for (uint32_t i = lane; i < n; i += 64) {
           const int64_t q = o + r0 + i;
@@ -937,20 +990,23 @@ __global__ void __launch_bounds__(WAVES * GROUPS * 64) seg_kernel(Params p) {
   extern __shared__ __align__(16) unsigned char smem[];
   SegLds<FILL>* lds = reinterpret_cast<SegLds<FILL>*>(smem);
   uint32_t* totals = reinterpret_cast<uint32_t*>(lds + WAVES * GROUPS);
-  ChromRec* tab = reinterpret_cast<ChromRec*>(totals + 2 * WAVES * GROUPS);
+  uint32_t* stops = totals + 2 * WAVES * GROUPS;
+  ChromRec* tab = reinterpret_cast<ChromRec*>(stops + 2 * (2 * WAVES + 1));
   for (int i = threadIdx.x; i <= p.n_chrom; i += blockDim.x) tab[i] = p.table[i];
   __syncthreads();
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t slot = WAVES == 1 ? (int64_t)blockIdx.x * GROUPS + wid : blockIdx.x;
   if (slot >= p.n_cells) return;
   const int64_t cell = p.order ? (int64_t)p.order[slot] : slot;
-  seg_cell<STRATEGY, WAVES, FILL, IdxT>(p, tab, &lds[wid], totals, cell, WAVES == 1 ? 0 : wid, lane);
+  seg_cell<STRATEGY, WAVES, FILL, IdxT>(p, tab, WAVES == 1 ? lds + wid : lds, totals, stops, cell,
+                                        WAVES == 1 ? 0 : wid, lane);
 }
 
 template <int STRATEGY, int WAVES, int GROUPS, bool FILL, typename IdxT>
 static int seg_launch(const Params& p, hipStream_t st) {
-  static_assert(sizeof(SegLds<FILL>) % 8 == 0 && (2 * WAVES * GROUPS * 4) % 8 == 0, "alignment of the table");
-  const size_t lds = (sizeof(SegLds<FILL>) + 8) * WAVES * GROUPS + sizeof(ChromRec) * (size_t)(p.n_chrom + 1);
+  static_assert(sizeof(SegLds<FILL>) % 8 == 0, "alignment of the table");
+  const size_t lds = (sizeof(SegLds<FILL>) + 8) * WAVES * GROUPS + 8 * (2 * WAVES + 1) +
+                     sizeof(ChromRec) * (size_t)(p.n_chrom + 1);
   if (lds > 160 * 1024) {
     set_error("chromosome table too large for LDS");
     return SNAPGPU_ERR_CAPACITY;

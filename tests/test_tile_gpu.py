@@ -362,3 +362,42 @@ def test_segments_hand_over_long_fragments(torch_gpu, length):
     for strategy in ("insertion", "paired-insertion", "fragment"):
         m, _, (cp, pos, ln) = _tile(torch_gpu, cells, cs, 100, [], None, None, strategy)
         _same(m, otile.tile_matrix(cp, pos, ln, cs, 100, [], None, None, strategy))
+
+
+@pytest.mark.parametrize("n_cells", [3, 1024, 8192])
+@pytest.mark.parametrize("strategy", ["insertion", "fragment", "paired-insertion", "single"])
+def test_segments_crowded_rows(torch_gpu, strategy, n_cells):
+    """Rows whose counts are carried through many segments: 20,000 fragments on 16 kb with lengths up
+    to 31 bins of 100 bases, one bin that holds many segments, and a chromosome's end amid them."""
+    rng = np.random.default_rng(n_cells)
+    cs = {"chr1": 16_000, "chr2": 3_000, "chr3": 9_000}
+    def row(n, a, b):
+        pos = np.sort(rng.integers(a, b, n))
+        end = np.where(pos < 16_000, 16_000, np.where(pos < 19_000, 19_000, 28_000))
+        return [(int(p), int(min(l, e - p))) for p, l, e in zip(pos, rng.integers(1, 3101, n), end)]
+    cells = [row(20_000, 0, 16_000), row(6_000, 12_000, 28_000),
+             [(5_000 + i // 2_000, 1 + (i * 37) % 3_050) for i in range(5_000)] + [(8_200, 100)] * 700]
+    cells += [row(int(k), 0, 28_000) for k in rng.integers(0, 20, n_cells - 3)]
+    m, _, (cp, pos, ln) = _tile(torch_gpu, cells, cs, 100, ["chr2"], None, None, strategy)
+    _same(m, otile.tile_matrix(cp, pos, ln, cs, 100, ["chr2"], None, None, strategy))
+
+
+def test_crowded_rows_take_no_longer(torch_gpu):
+    """The work is linear in the fragments, however they crowd (on 16 kb a look back over the
+    fragments within reach took ten times as long as the same number spread over 100 Mb)."""
+    torch = torch_gpu
+    from snapatac2_amd.pp import make_tile_matrix
+    rng = np.random.default_rng(1)
+    cs = {"chr1": 100_000_000}
+    times = {}
+    for width in (16_000, 90_000_000):
+        pos = np.sort(rng.integers(0, width, 50_000))
+        fr = _frags(torch, [[(int(p), int(l)) for p, l in zip(pos, rng.integers(30, 700, pos.size))]])[0]
+        for _ in range(6):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            make_tile_matrix(fr, cs)
+            b.record()
+            b.synchronize()
+            times[width] = min(times.get(width, 1e9), a.elapsed_time(b))
+    assert times[16_000] <= 3 * times[90_000_000], times
