@@ -154,7 +154,6 @@ constexpr int kChunk = 128;   // database points staged in LDS per step
 static_assert(kChunk == kWgQueries, "database chunk w must hold the queries of workgroup w");
 constexpr int kMaxLevels = 26;    // kd-tree depth bound (2^26 leaves >> INT32_MAX / 128)
 constexpr int kMaxSegs = 2 * 64 + 2;  // segments of leaves: two per cell and the ends
-constexpr int kSpreadSlice = 256;   // positions per block in the extent reduction (8 at a time)
 
 __device__ __forceinline__ unsigned int f2ord(float f) {
   const unsigned int u = __float_as_uint(f);
@@ -197,38 +196,40 @@ __global__ void kd_mm_init_kernel(unsigned int* mm, int64_t count) {
   if (t < count) mm[t] = (t & 1) ? 0u : 0xFFFFFFFFu;
 }
 
-// mm[node][c] = {min, max} (ordered-float bits) over the node's points.
-// Block (node i, slice s) covers positions node_begin[i] + s * kSpreadSlice ...
-__global__ void __launch_bounds__(256) kd_extent_kernel(const double* X, int d, int64_t ld,
-                                                        const uint32_t* order, const int64_t* nodes,
-                                                        int slices, unsigned int* mm) {
-  __shared__ unsigned int lmin[kDim], lmax[kDim];
-  const int64_t i = blockIdx.x / slices;
-  const int s = blockIdx.x % slices;
-  const int64_t b0 = nodes[2 * i], b1 = nodes[2 * i + 1];
-  const int64_t p0 = b0 + (int64_t)s * kSpreadSlice, p1 = min(b1, p0 + kSpreadSlice);
-  if (threadIdx.x < kDim) {
-    lmin[threadIdx.x] = 0xFFFFFFFFu;
-    lmax[threadIdx.x] = 0u;
+// mm[node][c] = {min, max} (ordered-float bits) over the node's points. A block takes
+// two leaves, 128 threads each: the launch grows with the points, whatever the sizes
+// of the segments.
+__global__ void __launch_bounds__(256) kd_extent_kernel(const double* X, int64_t n, int d, int64_t ld,
+                                                        const uint32_t* order, KdTables t, int level,
+                                                        unsigned int* mm) {
+  __shared__ unsigned int lmin[2][kDim], lmax[2][kDim];
+  __shared__ int64_t node[2];  // -1: no points, or nothing to split
+  const int c = threadIdx.x & 31, u = threadIdx.x >> 5, half = u >> 2;
+  const int64_t leaf = 2 * (int64_t)blockIdx.x + half;
+  const int64_t p0 = leaf * kChunk, p1 = min(n, p0 + kChunk);
+  if (threadIdx.x < 2 * kDim) {
+    lmin[u][c] = 0xFFFFFFFFu;
+    lmax[u][c] = 0u;
   }
+  bool done = true;
+  const int64_t id = p0 < n ? (int64_t)kd_node(t, (int32_t)leaf, level, &done) : 0;
+  if ((threadIdx.x & 127) == 0) node[half] = done ? -1 : id;
   __syncthreads();
-  if (p0 < p1) {
-    const int c = threadIdx.x & 31;
+  if (!done && c < d) {
     unsigned int mn = 0xFFFFFFFFu, mx = 0u;
-    if (c < d) {
-      for (int64_t p = p0 + (threadIdx.x >> 5); p < p1; p += blockDim.x / 32) {
-        const unsigned int o = f2ord((float)X[(int64_t)order[p] * ld + c]);
-        mn = min(mn, o);
-        mx = max(mx, o);
-      }
-      atomicMin(&lmin[c], mn);
-      atomicMax(&lmax[c], mx);
+    for (int64_t p = p0 + (u & 3); p < p1; p += 4) {
+      const unsigned int o = f2ord((float)X[(int64_t)order[p] * ld + c]);
+      mn = min(mn, o);
+      mx = max(mx, o);
     }
+    const int to = half != 0 && node[0] == node[1] ? 0 : half;
+    atomicMin(&lmin[to][c], mn);
+    atomicMax(&lmax[to][c], mx);
   }
   __syncthreads();
-  if (p0 < p1 && threadIdx.x < d) {
-    atomicMin(&mm[(i * kDim + threadIdx.x) * 2], lmin[threadIdx.x]);
-    atomicMax(&mm[(i * kDim + threadIdx.x) * 2 + 1], lmax[threadIdx.x]);
+  if (u < 2 && c < d && node[u] >= 0 && !(u == 1 && node[0] == node[1])) {
+    atomicMin(&mm[(node[u] * kDim + c) * 2], lmin[u][c]);
+    atomicMax(&mm[(node[u] * kDim + c) * 2 + 1], lmax[u][c]);
   }
 }
 
@@ -1436,7 +1437,6 @@ struct Workspace {
   uint64_t *keys, *keys2;
   uint32_t *order0, *order;
   unsigned int* mm;
-  int64_t* kd_nodes;
   float *pivot, *margin;
   int32_t *leaf_cell, *wg_order, *kd_tab;
   int64_t* cell_begin;
@@ -1476,7 +1476,6 @@ static int64_t layout(int64_t n, Workspace* w, char* base) {
   t.order = (uint32_t*)take(n * 4);
   const int64_t nl = ceil_div(n, kChunk);
   t.mm = (unsigned int*)take((nl + kMaxSegs) * kDim * 2 * 4);
-  t.kd_nodes = (int64_t*)take((2 * nl + kMaxSegs * kMaxLevels) * 2 * 8);
   t.kd_tab = (int32_t*)take((nl + kMaxSegs * (kMaxLevels + 3)) * 4);
   t.leaf_cell = (int32_t*)take(nl * 4);
   t.wg_order = (int32_t*)take(nl * 4);
@@ -1543,7 +1542,7 @@ int snapgpu_knn(const double* d_X, int64_t n, int32_t d, int64_t ld, int32_t k, 
                mode == kModeBF16 ? kEpsBF16 : kEpsFP32, (flags & 1) ? 1 : 0,
                d_nbr, d_dist, w.fail_rows, w.fail_count};
   // host tables of the order: they outlive their copies to the device (synchronised below)
-  std::vector<int64_t> tab, cell_begin(kCells + 1, 0);
+  std::vector<int64_t> cell_begin(kCells + 1, 0);
   std::vector<int32_t> tab32, leaf_cell, wg_order;
   if (mode == kModeBF16) {
     // spatial order of the queries, per-workgroup centres, centred LDS-staged MFMA tiles
@@ -1596,43 +1595,20 @@ int snapgpu_knn(const double* d_X, int64_t n, int32_t d, int64_t ld, int32_t k, 
     for (int s = 0; s < segs; ++s) std::fill(tab32.begin() + seg_begin[s], tab32.begin() + seg_begin[s + 1], s);
     tab32.insert(tab32.end(), seg_begin.begin(), seg_begin.end());
     tab32.insert(tab32.end(), depth.begin(), depth.end());
-    // tab: positions of the nodes, level by level
-    std::vector<int64_t> level_off(levels + 1, 0);
-    for (int l = 0; l < levels; ++l) {
-      level_off[l] = (int64_t)tab.size() / 2;
+    std::vector<int64_t> level_nodes(levels, 0);
+    for (int l = 0; l < levels; ++l)
       for (int s = 0; s < segs; ++s) {
-        tab32.push_back((int32_t)((int64_t)tab.size() / 2 - level_off[l]));
-        if (l >= depth[s]) {
-          tab.insert(tab.end(), 2, 0);
-          continue;
-        }
-        for (int64_t id = 0; id < ((int64_t)1 << l); ++id) {
-          int64_t a = seg_begin[s], b = seg_begin[s + 1];
-          for (int q = l - 1; q >= 0; --q) {
-            const int64_t m = a + (b - a + 1) / 2;
-            if ((id >> q) & 1) a = m; else b = m;
-          }
-          tab.push_back(std::min(a * kChunk, n));
-          tab.push_back(std::min(b * kChunk, n));
-        }
+        tab32.push_back((int32_t)level_nodes[l]);
+        level_nodes[l] += l < depth[s] ? (int64_t)1 << l : 1;
       }
-    }
-    level_off[levels] = (int64_t)tab.size() / 2;
     SG_HIP(hipMemcpyAsync(w.kd_tab, tab32.data(), tab32.size() * 4, hipMemcpyHostToDevice, st));
-    if (!tab.empty())
-      SG_HIP(hipMemcpyAsync(w.kd_nodes, tab.data(), tab.size() * 8, hipMemcpyHostToDevice, st));
     const KdTables kt{w.kd_tab, w.kd_tab + nl, w.kd_tab + nl + segs + 1, w.kd_tab + nl + 2 * segs + 1, segs};
-    int64_t widest = 0;
-    for (int s = 0; s < segs; ++s) widest = std::max<int64_t>(widest, seg_begin[s + 1] - seg_begin[s]);
     for (int l = 0; l < levels; ++l) {
-      const int64_t nodes = level_off[l + 1] - level_off[l];
-      const int64_t max_size = ceil_div(widest, (int64_t)1 << l) * kChunk;
-      const int slices = (int)std::max<int64_t>(1, ceil_div(max_size, kSpreadSlice));
+      const int64_t nodes = level_nodes[l];
       int bits = 1;
       while (((int64_t)1 << bits) < nodes) ++bits;
       kd_mm_init_kernel<<<(unsigned)ceil_div(nodes * kDim * 2, 256), 256, 0, st>>>(w.mm, nodes * kDim * 2);
-      kd_extent_kernel<<<(unsigned)(nodes * slices), 256, 0, st>>>(d_X, d, ld, w.order,
-                                                                  w.kd_nodes + 2 * level_off[l], slices, w.mm);
+      kd_extent_kernel<<<(unsigned)ceil_div(nl, 2), 256, 0, st>>>(d_X, n, d, ld, w.order, kt, l, w.mm);
       kd_key_kernel<<<(unsigned)ceil_div(n, 256), 256, 0, st>>>(d_X, n, d, ld, w.order, kt, l, w.mm, w.keys,
                                                                w.order0);
       SG_LAUNCH_CHECK();

@@ -189,7 +189,7 @@ def test_candidates_far_from_the_centre(torch_gpu):
 
 @pytest.mark.parametrize("kind,n,d", [("clusters", 16383, 30), ("clusters", 16385, 30), ("clusters", 33001, 7),
                                       ("one cluster", 25000, 30), ("line", 40000, 1), ("duplicates", 20001, 4),
-                                      ("constant", 16400, 3), ("scales", 30000, 5)])
+                                      ("constant", 16400, 3), ("scales", 30000, 5), ("dominant", 30001, 6)])
 def test_cells(torch_gpu, kind, n, d):
     """From 16,384 rows on (128 leaves) the rows are ordered by cells and chunks are skipped by
     the planes between them: the graph of a run that skips nothing, and the oracle's rows."""
@@ -201,6 +201,7 @@ def test_cells(torch_gpu, kind, n, d):
          "line": lambda: rng.random((n, 1)),
          "duplicates": lambda: rng.integers(0, 9, (n, d)).astype(np.float64),
          "constant": lambda: np.full((n, d), 0.25),
+         "dominant": lambda: rng.standard_normal((n, d)) + 40.0 * rng.integers(0, 4, (n, d)) * (rng.random((n, 1)) < 0.1),
          "scales": lambda: rng.standard_normal((n, d)) * 10.0 ** rng.integers(-4, 5, n)[:, None]}[kind]()
     g = nearest_neighbour_graph(X, k)
     full = nearest_neighbour_graph(X, k, prune=False)
