@@ -12,10 +12,10 @@
 //     mode forms them as it stages a chunk.
 //  2. candidates. BF16 mode: the points are put in kd-tree leaf order (leaves of
 //     128), each leaf is shifted by its own centre, and a workgroup of 8 waves
-//     (128 queries = one leaf) streams database leaves through LDS, each as two
-//     bf16 terms (x = hi + lo + O(2^-18 x)) multiplied with three
-//     v_mfma_f32_16x16x32_bf16 per 16x16 tile (hi hi, hi lo, lo hi; fp32
-//     accumulation). A leaf whose bounding sphere lies beyond every query's
+//     (128 queries = one leaf) streams database leaves through LDS, each as three
+//     bf16 terms (x = hi + mid + lo, exactly) multiplied with six
+//     v_mfma_f32_16x16x32_bf16 per 16x16 tile (all products but mid lo, lo mid and
+//     lo lo; fp32 accumulation). A leaf whose bounding sphere lies beyond every query's
 //     current threshold is skipped (the threshold is kept in the certificate, so
 //     skipping stays exact).
 //     FP32 mode: SIMT FMAs over every point in the original order. In both,
@@ -52,24 +52,27 @@ constexpr int kMaxData = 30;  // data dimensions supported
 constexpr int kList = 32;     // candidates kept per lane (stripe)
 constexpr int kCand = 4 * kList;  // candidates per query
 constexpr int kMaxK = 100;
-// Up to kSmallK neighbours a lane of the BF16 path keeps half as many candidates: its
-// stripe then holds more than 16 of the 25 nearest for one query in 50,000 (binomial,
-// four stripes), and such rows go to the second tier as any other that is not certified.
+// Up to kSmallK neighbours a lane of the BF16 path keeps half as many candidates. A row
+// is not certified where a stripe holds 16 of the 25 nearest (its 16th bounds what it
+// left out), or 15 in the query's own stripe, whose list the query itself is in: one
+// query in 2,900 (binomial, four stripes). Such rows go to the second tier as any other.
 constexpr int kSmallK = 25, kSmallList = 16;
 
 enum Mode : int32_t { kModeFP32 = 0, kModeBF16 = 1 };
 
 // Error constants c of the approximate d^2 (see the certificate above):
 // |approx - exact| <= c * (|x||q| + |x|^2 + |q|^2).
-// BF16 (two-term split, three products): each term rounds to 2^-9 of what it
-// holds, so lo lo' and the two remainders leave out <= 3 * 2^-18 |x||q|, and the
-// remainder of the |x|^2 coordinate (times an exact -1/2) 2^-19 |x|^2; fp32
-// accumulation of 96 terms adds <= 96 * 2^-24 (|x||q| + |x|^2 / 2); all doubled by
-// d^2 = |q|^2 - 2s, plus fp32 rounding of the inputs and of the norms (32 * 2^-24):
-// 3.5e-5 |x||q| + 1.2e-5 |x|^2 + 2e-6 |q|^2, so c = 4e-5. A third term and three
-// more products would only take this to 3e-5, most of it the accumulation.
+// BF16 (three-term split, six products): a bf16 value has 8 significant bits, so for
+// 2^e <= |x| < 2^(e+1) the first term leaves at most 2^(e-8), the second 2^(e-17), and
+// what is left of an fp32 value then (a multiple of 2^(e-23)) is the third. The omitted
+// products are mid lo', lo mid' and lo lo', 2^-24 |x||q| together; -1/2 is one term, so
+// none of the |x|^2 coordinate's is. fp32 accumulation of 192 terms adds at most
+// 1.02 * 192 * 2^-24 (|x||q| + |x|^2 / 2). All doubled by d^2 = |q|^2 - 2s, plus fp32
+// rounding of the inputs and of the norms: 2.4e-5 |x||q| + 1.3e-5 |x|^2 + 2e-6 |q|^2,
+// so c = 3e-5. (Two terms and three products leave 2^-15 |x||q|, which c = 4e-5 would
+// still cover; they send twice as many rows to the second tier.)
 // FP32: 32 sequential FMAs (<= 32 * 2^-24), doubled, plus input rounding: c = 1e-5.
-constexpr double kEpsBF16 = 4.0e-5;
+constexpr double kEpsBF16 = 3.0e-5;
 constexpr double kEpsFP32 = 1.0e-5;
 
 __device__ __forceinline__ __bf16 to_bf16(float x) { return (__bf16)x; }
@@ -277,7 +280,8 @@ __global__ void kd_key_kernel(const double* X, int64_t n, int d, int64_t ld, con
 // a's side (negative beyond it), so d(x, y) is at least the smallest such distance
 // in the one chunk plus the smallest in the other, whichever cells their points
 // really belong to. 1M clustered rows of 30 dimensions, k = 50: the candidate
-// kernel 115 -> 55 ms (39% of the chunk pairs visited without cells).
+// kernel 115 -> 55 ms with two bf16 terms, 62 with three (39% of the chunk pairs
+// visited without cells).
 constexpr int kCells = 64;
 constexpr int kLeavesPerCell = 64;
 constexpr int kCellSample = 8192;
@@ -493,9 +497,11 @@ __device__ __forceinline__ int64_t visit_chunk(int64_t v, int64_t w, int64_t nwg
   return (k >= 0 && k < nwg) ? k : -1;
 }
 
-__device__ __forceinline__ void split2(float x, __bf16& h, __bf16& l) {
+__device__ __forceinline__ void split3(float x, __bf16& h, __bf16& m, __bf16& l) {
   h = to_bf16(x);
-  l = to_bf16(x - (float)h);
+  const float r = x - (float)h;
+  m = to_bf16(r);
+  l = to_bf16(r - (float)m);
 }
 
 // Workgroup = 8 waves = 128 consecutive sorted queries sharing one centre.
@@ -509,16 +515,17 @@ __device__ __forceinline__ void split2(float x, __bf16& h, __bf16& l) {
 // Thresholds only shrink, so every skipped point has exact d^2 > the final
 // threshold: the certificate of the finalize step holds for it as for a point
 // that was seen and not kept. Processed chunks are shifted by
-// the centre, given their augmented coordinate |x - c|^2, split into two
+// the centre, given their augmented coordinate |x - c|^2, split into three
 // bf16 terms and staged in LDS; every wave then runs its 16 x 16 MFMA tiles.
 //
 // The kernel is bound by instruction issue around its MFMA, so a tile costs what
-// it must: two LDS reads, three MFMA, the largest of a lane's four values against
+// it must: three LDS reads, six MFMA, the largest of a lane's four values against
 // its threshold and one branch. The queue (below) lies in LDS, where an append is
 // one store, and its flush is a loop, which also keeps the kernel's code small
-// enough for a first pass not to wait for its instructions. 1M clustered rows of
-// 30 dimensions, k = 50 (24M chunk pairs): 347 ms with three terms, six MFMA and
-// register queues, 115 ms so; 2,777 rows: 774 and 255 us.
+// enough for a first pass not to wait for its instructions. 2,777 rows: 774 us with
+// register queues, 259 so. 1M clustered rows of 30 dimensions, k = 50 (the chunks that
+// the planes between the cells leave): 62 ms; two terms and three MFMA took 55, and the
+// operands would hold 16 bits where the FP32 path's hold 24.
 //
 // Accepted candidates of the candidate kernels wait in a per-lane queue of kQueue
 // entries and enter the sorted list together. list_insert runs for the whole
@@ -592,7 +599,7 @@ __device__ __forceinline__ void lds_queue_flush(const float2 (*e)[kWgWaves * 64]
 }
 
 // Entries of a lane's LDS queue: two workgroups share a CU's 160 KB.
-constexpr int kCandQueue = 15;
+constexpr int kCandQueue = 13;
 
 // Augmented coordinate of the positions past n: their s lies below any real
 // point's, so they are not kept unless a list has room (and then written as -1).
@@ -600,7 +607,7 @@ constexpr float kPadNorm = 1e38f;
 
 template <int LIST>
 __global__ void __launch_bounds__(kWgWaves * 64, 4) cand_centred_kernel(CentredParams P) {
-  __shared__ __align__(16) __bf16 As[2][kChunk][kDim];
+  __shared__ __align__(16) __bf16 As[3][kChunk][kDim];
   __shared__ float2 queue[kCandQueue][kWgWaves * 64];
   __shared__ float cen[kDim];
   __shared__ float red[kWgWaves];
@@ -615,8 +622,8 @@ __global__ void __launch_bounds__(kWgWaves * 64, 4) cand_centred_kernel(CentredP
   __syncthreads();
   const int64_t qi = wg * kWgQueries + wv * 16 + j;  // sorted position
   const bool qvalid = qi < P.n;
-  // query operand: (q - c, -1/2 at dim 30), split in two bf16 terms
-  bf16x8 bq_h, bq_l;
+  // query operand: (q - c, -1/2 at dim 30), split in three bf16 terms
+  bf16x8 bq_h, bq_m, bq_l;
   float part = 0.f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
@@ -626,9 +633,10 @@ __global__ void __launch_bounds__(kWgWaves * 64, 4) cand_centred_kernel(CentredP
     if (qvalid && c < P.d) v = (float)(P.xs[qi * kDim + c] - (double)cen[c]);
     if (c == kMaxData) v = -0.5f;
     if (c < P.d) part = fmaf(v, v, part);
-    __bf16 h, l;
-    split2(v, h, l);
+    __bf16 h, m, l;
+    split3(v, h, m, l);
     bq_h[e] = h;
+    bq_m[e] = m;
     bq_l[e] = l;
   }
   part += __shfl_xor(part, 16, 64);
@@ -647,10 +655,6 @@ __global__ void __launch_bounds__(kWgWaves * 64, 4) cand_centred_kernel(CentredP
   unsigned long long visited = 0;
   // staging roles: thread t -> point t/4, dims (t%4)*8 .. +7
   const int sp = tid >> 2, sq = tid & 3;
-  // this thread's dimensions of the centre (zero past d, as the rows are)
-  float cs[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) cs[e] = cen[sq * 8 + e];
   // the first batch is the workgroup's own chunk alone, so that the thresholds
   // are finite when the other chunks are tested
   for (int64_t v0 = 0, bs = 1; v0 < 2 * P.n_wg; v0 += bs, bs = 64) {
@@ -722,22 +726,24 @@ __global__ void __launch_bounds__(kWgWaves * 64, 4) cand_centred_kernel(CentredP
         float ps = 0.f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          v[e] = (float)((e & 1 ? xr[e / 2].y : xr[e / 2].x) - (double)cs[e]);
+          v[e] = (float)((e & 1 ? xr[e / 2].y : xr[e / 2].x) - (double)cen[sq * 8 + e]);  // zero past d
           ps = fmaf(v[e], v[e], ps);
         }
         ps += __shfl_xor(ps, 1, 64);
         ps += __shfl_xor(ps, 2, 64);
         if (sq == 3) v[6] = c0 + sp < P.n ? ps : kPadNorm;  // dim 30 = |x - c|^2
-        bf16x8 th, tl;
+        bf16x8 th, tm, tl;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          __bf16 h, l;
-          split2(v[e], h, l);
+          __bf16 h, mid, l;
+          split3(v[e], h, mid, l);
           th[e] = h;
+          tm[e] = mid;
           tl[e] = l;
         }
         *reinterpret_cast<bf16x8*>(&As[0][sp][sq * 8]) = th;
-        *reinterpret_cast<bf16x8*>(&As[1][sp][sq * 8]) = tl;
+        *reinterpret_cast<bf16x8*>(&As[1][sp][sq * 8]) = tm;
+        *reinterpret_cast<bf16x8*>(&As[2][sp][sq * 8]) = tl;
       }
       __syncthreads();
       if (m != 0) prefetch(m);
@@ -748,10 +754,14 @@ __global__ void __launch_bounds__(kWgWaves * 64, 4) cand_centred_kernel(CentredP
         for (int h = 0; h < 2; ++h) {
           const int row = (tt + h) * 16 + j;
           const bf16x8 ah = *reinterpret_cast<const bf16x8*>(&As[0][row][g * 8]);
-          const bf16x8 al = *reinterpret_cast<const bf16x8*>(&As[1][row][g * 8]);
+          const bf16x8 am = *reinterpret_cast<const bf16x8*>(&As[1][row][g * 8]);
+          const bf16x8 al = *reinterpret_cast<const bf16x8*>(&As[2][row][g * 8]);
           acc[h] = f32x4{0.f, 0.f, 0.f, 0.f};
           acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bq_h, acc[h], 0, 0, 0);
+          acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(am, bq_m, acc[h], 0, 0, 0);
           acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bq_l, acc[h], 0, 0, 0);
+          acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(am, bq_h, acc[h], 0, 0, 0);
+          acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bq_m, acc[h], 0, 0, 0);
           acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bq_h, acc[h], 0, 0, 0);
         }
         const float th = L[LIST - 1];
