@@ -616,7 +616,8 @@ int snapgpu_frag_index(const uint8_t* d_text, int64_t n_bytes, int64_t n_lines, 
                        const void* d_whitelist, const snapgpu_frag_options* opt, void* d_ws, int64_t ws_bytes,
                        snapgpu_frag_summary* h_summary, void* stream);
 /* The same with the workspace that snapgpu_frag_count_lines has just filled for this
- * text (NULL: the lines are counted again). */
+ * text (NULL: the lines are counted again). One whose counts are not this text's is
+ * SNAPGPU_ERR_ARG. */
 int snapgpu_frag_index_counted(const uint8_t* d_text, int64_t n_bytes, int64_t n_lines, const void* d_count_ws,
                                int64_t count_ws_bytes, const void* d_chroms, const void* d_whitelist,
                                const snapgpu_frag_options* opt, void* d_ws, int64_t ws_bytes,

@@ -99,6 +99,7 @@ struct Counters {
   unsigned int any_bad;         // a whitelisted group holds a record count_fragments cannot convert
   unsigned int max_size;        // largest end - start (low 32 bits) over kept records
   unsigned long long n_groups;  // distinct barcodes of unsorted input
+  unsigned int recount;         // a block's newlines are not as many as were counted
 };
 
 // How the records were sorted, for the kernels that read the result: the key holds
@@ -279,11 +280,12 @@ __global__ void __launch_bounds__(kThreads) nl_count_kernel(const uint8_t* __res
 }
 
 // line_start[0] = 0 and line_start[k + 1] = (position of newline k) + 1.
-// blk_incl: inclusive scan of the per-block newline counts; n_lines bounds the writes
-// (a text that has changed since it was counted).
+// blk_incl: inclusive scan of the per-block newline counts. A block that finds another
+// number (a text that has changed since it was counted, a workspace of another text)
+// says so, and n_lines bounds the writes: where none does, every entry is written.
 __global__ void __launch_bounds__(kThreads) nl_index_kernel(const uint8_t* __restrict__ text, int64_t n,
                                                             const int64_t* __restrict__ blk_incl, int64_t n_lines,
-                                                            int64_t* __restrict__ line_start) {
+                                                            int64_t* __restrict__ line_start, Counters* cnt) {
   __shared__ int64_t wsum[kThreads / 64];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int64_t w0 = (int64_t)blockIdx.x * kThreads * kRounds;
@@ -307,12 +309,13 @@ __global__ void __launch_bounds__(kThreads) nl_index_kernel(const uint8_t* __res
     while (m) {
       const int k = __ffs(m) - 1;
       m &= m - 1;
-      if (o < n_lines) line_start[1 + o] = wi * 16 + k + 1;
+      if ((uint64_t)o < (uint64_t)n_lines) line_start[1 + o] = wi * 16 + k + 1;
       ++o;
     }
     base += total;
     __syncthreads();
   }
+  if (threadIdx.x == 0 && base != blk_incl[blockIdx.x]) atomicOr(&cnt->recount, 1u);
 }
 
 // ---------------------------------------------------------------------------
@@ -1597,25 +1600,28 @@ int snapgpu_frag_index_counted(const uint8_t* d_text, int64_t n_bytes, int64_t n
     if (rc) return rc;
     nl = blk;
   }
-  // line_start holds n_lines + 1 entries: check n_lines before writing them
-  int64_t n_nl = 0;
-  uint8_t last = 0;
-  SG_HIP(hipMemcpyAsync(&n_nl, nl + nb - 1, 8, hipMemcpyDeviceToHost, st));
-  SG_HIP(hipMemcpyAsync(&last, d_text + n_bytes - 1, 1, hipMemcpyDeviceToHost, st));
-  SG_HIP(hipStreamSynchronize(st));
-  SG_ARG(n_lines == n_nl + (last != '\n' ? 1 : 0), "n_lines does not match the text");
-  nl_index_kernel<<<(unsigned)nb, kThreads, 0, st>>>(d_text, n_bytes, nl, n_lines, line_start);
-  SG_LAUNCH_CHECK();
-  const int64_t sentinel = n_bytes + 1;  // end of a last line without '\n'
-  if (last != '\n') SG_HIP(hipMemcpyAsync(line_start + n_lines, &sentinel, 8, hipMemcpyHostToDevice, st));
-
-  // 2. parse
   Counters c0{};
   c0.err = ~0ull;
   c0.first = ~0ull;
   c0.bad = ~0ull;
   c0.dup = ~0ull;
   SG_HIP(hipMemcpyAsync(C, &c0, sizeof(Counters), hipMemcpyHostToDevice, st));
+  nl_index_kernel<<<(unsigned)nb, kThreads, 0, st>>>(d_text, n_bytes, nl, n_lines, line_start, C);
+  SG_LAUNCH_CHECK();
+  // nothing reads line_start before the host knows that it is whole
+  int64_t n_nl = 0;
+  uint8_t last = 0;
+  unsigned int recount = 0;
+  SG_HIP(hipMemcpyAsync(&recount, &C->recount, 4, hipMemcpyDeviceToHost, st));
+  SG_HIP(hipMemcpyAsync(&n_nl, nl + nb - 1, 8, hipMemcpyDeviceToHost, st));
+  SG_HIP(hipMemcpyAsync(&last, d_text + n_bytes - 1, 1, hipMemcpyDeviceToHost, st));
+  SG_HIP(hipStreamSynchronize(st));
+  SG_ARG(n_lines == n_nl + (last != '\n' ? 1 : 0), "n_lines does not match the text");
+  SG_ARG(recount == 0, "the count workspace is not this text's");
+  const int64_t sentinel = n_bytes + 1;  // end of a last line without '\n'
+  if (last != '\n') SG_HIP(hipMemcpyAsync(line_start + n_lines, &sentinel, 8, hipMemcpyHostToDevice, st));
+
+  // 2. parse
   ParseOut po{at<uint32_t>(w, Lo.pos), at<uint32_t>(w, Lo.size), at<uint32_t>(w, Lo.cnt), at<uint8_t>(w, Lo.flags),
               at<uint64_t>(w, Lo.bc), opt->sorted_by_barcode ? nullptr : at<uint64_t>(w, Lo.bch)};
   const int64_t lb = ceil_div(n_lines, kLineBlock);

@@ -123,3 +123,41 @@ def test_lines_counted_again(torch_gpu, monkeypatch, last):
     off[0] = -1
     with pytest.raises(Exception, match="n_lines"):
         _gpu(text, {"chr1": 6000}, min_num_fragments=0)
+
+
+@pytest.mark.parametrize("change", ["fewer", "moved", "more", "zeros", "ones"])
+def test_count_workspace_of_another_text(torch_gpu, change):
+    """A text that changed since its lines were counted, or a workspace that holds something
+    else, is refused before anything reads the line starts."""
+    import ctypes as C
+    torch = torch_gpu
+    from snapatac2_amd import _lib
+    L = _lib.lib()
+    line = b"chr1\t%05d\t99999\tcell\n"
+    text = np.frombuffer(b"".join(line % i for i in range(8000)), np.uint8).copy()
+    size = text.size
+    assert size > 2 * 65536
+    pad = torch.zeros(size + 16, dtype=torch.uint8, device="cuda")
+    pad[:size] = torch.from_numpy(text).cuda()
+    ws = torch.empty(L.snapgpu_frag_count_workspace_bytes(size), dtype=torch.uint8, device="cuda")
+    n = C.c_int64(0)
+    st = _lib.stream_ptr()
+    _lib.check(L.snapgpu_frag_count_lines(pad.data_ptr(), size, ws.data_ptr(), ws.numel(), C.byref(n), st))
+    assert n.value == 8000
+    w = len(line % 0)
+    if change in ("fewer", "moved"):
+        pad[w - 1] = ord("x")  # one newline less in the first block of 64 KiB
+    if change in ("more", "moved"):
+        pad[size - 5] = 10     # one more in the last
+    if change == "zeros":
+        ws.zero_()
+    if change == "ones":
+        ws.fill_(255)
+    from snapatac2_amd.pp._import import _name_table
+    d_tab = torch.from_numpy(_name_table(["chr1"], [100_000], [0])).cuda()
+    iws = torch.zeros(L.snapgpu_frag_workspace_bytes(size, n.value), dtype=torch.uint8, device="cuda")
+    opt, summ = _lib.FragOptions(0, 0, 0, 1, 0), _lib.FragSummary()
+    rc = L.snapgpu_frag_index_counted(pad.data_ptr(), size, n.value, ws.data_ptr(), ws.numel(), d_tab.data_ptr(), None,
+                                      C.byref(opt), iws.data_ptr(), iws.numel(), C.byref(summ), st)
+    assert rc == _lib.ERR_ARG
+    assert b"count workspace" in L.snapgpu_last_error() or b"n_lines" in L.snapgpu_last_error()
