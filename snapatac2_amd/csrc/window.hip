@@ -49,10 +49,6 @@ constexpr int kChunk = 64;                         // build chunk of a row
 constexpr int kThreads = 1024;
 constexpr int kQuads = kThreads / 4;
 constexpr int kMaxWindows = 16384;                 // LDS counters of the build (64 KB)
-#ifndef SNAPGPU_WINDOW_PRE
-#define SNAPGPU_WINDOW_PRE 16
-#define SNAPGPU_WINDOW_STEP 4
-#endif
 constexpr uint32_t kFlag = 1u << (kWinBits + 11);  // after the column and the 11-bit slot
 static_assert(kWinBits + 12 <= 24, "column, slot and flag must stay below the count byte");
 
@@ -300,7 +296,21 @@ __device__ __forceinline__ void store_row(float4 t, int64_t row, int q, const fl
   }
 }
 
-template <int EPI>
+// PRE: entries of a quad's chunk loaded a window ahead (the rest follow one step after
+// the other), kStep of them taken at once. Per application, 16 and 24 ahead, by the
+// average chunk: 7 entries 9.5 and 9.9 ms, 10 entries 12.0 and 12.2, 12.6 entries 14.4 and
+// 14.6, 15.5 entries 17.4 and 17.3 (800,000 cells), 21.9 and 21.6 (a million), 19 entries
+// 21.2 and 21.4, 30 entries 8.3 and 8.5, 43 entries 14.9 and 15.3. 24 pay where most chunks
+// lie between the two: a million cells with peaks, 15.8 entries, 23.4 and 22.9 (steps of 8,
+// 24 ahead: 22.9 there, 3 to 9% slower than 16 and 4 up to 12.6 entries).
+constexpr int kStep = 4;
+
+static bool far_ahead(const snapgpu_window_layout& L) {
+  const double chunk = (double)L.n_entries / ((double)L.n_blocks * (double)L.n_windows * kQuads);
+  return chunk >= 14.0 && chunk < 18.0;
+}
+
+template <int EPI, int PRE>
 __global__ void __launch_bounds__(kThreads) product_kernel(
     const uint32_t* __restrict__ ent, const int64_t* __restrict__ bstart, const uint32_t* __restrict__ qoff,
     int64_t nw, const int64_t* __restrict__ block_row, const uint32_t* __restrict__ row_slot,
@@ -321,16 +331,11 @@ __global__ void __launch_bounds__(kThreads) product_kernel(
     const int64_t w1 = min(nw, w0 + (stop - at));
     for (int i = tid; i < kSlots * 4; i += kThreads) acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     __syncthreads();
-    // Window w + 2's bounds and window w + 1's first kPre entries are loaded while
+    // Window w + 2's bounds and window w + 1's first PRE entries are loaded while
     // window w is summed, so neither dependent load (bounds, then entries) sits
     // on a window's critical path. Entries past a chunk's end read as 0 (no piece
     // start, count 0): they add 0 * z to the open piece, z being a row of the
-    // same window. A quad's chunk is nine entries on average at 891 million
-    // entries in 778 blocks x 489 windows, so what is taken at once is small: per
-    // application 11.93 ms with 24 loaded ahead and 8 at a time, 11.71 with 16 and
-    // 8, 11.28 with 16 and 4, 11.39 with 8 and 4; 1.9 billion in 982 blocks (sixteen
-    // a chunk) 22.14 with 24 and 8, 21.56 with 24 and 4, 21.84 with 16 and 4.
-    constexpr int kPre = SNAPGPU_WINDOW_PRE, kStep = SNAPGPU_WINDOW_STEP;
+    // same window.
     const int64_t bq0 = blk * nw;
     int64_t bs = bstart[bq0 + w0];
     uint32_t p0 = qoff[(bq0 + w0) * (kQuads + 1) + quad], p1 = qoff[(bq0 + w0) * (kQuads + 1) + quad + 1];
@@ -341,15 +346,15 @@ __global__ void __launch_bounds__(kThreads) product_kernel(
       p01 = qoff[(bq0 + w0 + 1) * (kQuads + 1) + quad];
       p11 = qoff[(bq0 + w0 + 1) * (kQuads + 1) + quad + 1];
     }
-    uint32_t vpre[kPre];
+    uint32_t vpre[PRE];
 #pragma unroll
-    for (int u = 0; u < kPre; ++u) vpre[u] = p0 + u < p1 ? ent[bs + p0 + u] : 0u;
+    for (int u = 0; u < PRE; ++u) vpre[u] = p0 + u < p1 ? ent[bs + p0 + u] : 0u;
     for (int64_t w = w0; w < w1; ++w) {
       const bool more1 = w + 1 < w1, more2 = w + 2 < w1;
       // window w + 1's first entries, window w + 2's bounds
-      uint32_t vn[kPre];
+      uint32_t vn[PRE];
 #pragma unroll
-      for (int u = 0; u < kPre; ++u) vn[u] = (more1 && p01 + u < p11) ? ent[bs1 + p01 + u] : 0u;
+      for (int u = 0; u < PRE; ++u) vn[u] = (more1 && p01 + u < p11) ? ent[bs1 + p01 + u] : 0u;
       int64_t bs2 = 0;
       uint32_t p02 = 0, p12 = 0;
       if (more2) {
@@ -364,7 +369,7 @@ __global__ void __launch_bounds__(kThreads) product_kernel(
       uint32_t slot = 0;
       bool open = false;  // the chunk starts at a piece start, so its first entry opens one
 #pragma unroll
-      for (int h = 0; h < kPre; h += kStep) {
+      for (int h = 0; h < PRE; h += kStep) {
         if (p0 + h < p1) {
           float4 z[kStep];
 #pragma unroll
@@ -374,7 +379,7 @@ __global__ void __launch_bounds__(kThreads) product_kernel(
           for (int u = 0; u < kStep; ++u) gather_entry(acc, q, vpre[h + u], z[u], open, slot, a);
         }
       }
-      for (uint32_t p = p0 + kPre; p < p1; p += kStep) {
+      for (uint32_t p = p0 + PRE; p < p1; p += kStep) {
         uint32_t v[kStep];
         float4 z[kStep];
 #pragma unroll
@@ -394,7 +399,7 @@ __global__ void __launch_bounds__(kThreads) product_kernel(
       p01 = p02;
       p11 = p12;
 #pragma unroll
-      for (int u = 0; u < kPre; ++u) vpre[u] = vn[u];
+      for (int u = 0; u < PRE; ++u) vpre[u] = vn[u];
     }
     // epilogue: 4 lanes per row
     const int64_t r0 = block_row[blk], r1 = block_row[blk + 1];
@@ -456,7 +461,8 @@ static void product(const snapgpu_window_layout& L, const float* dense, const fl
                    spare_rows >= 2 * (int64_t)kShares * kSlots;
   const int64_t full = cut ? L.n_blocks - rest : L.n_blocks;
   float4* part = reinterpret_cast<float4*>(spare);
-  product_kernel<EPI><<<(unsigned)(full + (cut ? kShares : 0)), kThreads, 0, st>>>(
+  const auto kernel = far_ahead(L) ? product_kernel<EPI, 24> : product_kernel<EPI, 16>;
+  kernel<<<(unsigned)(full + (cut ? kShares : 0)), kThreads, 0, st>>>(
       L.ent, L.bucket_start, L.quad_off, L.n_windows, L.block_row, L.row_slot, dense, scale, out32, V, ldv, dinv, Y,
       ldy, b, full, L.n_blocks, part);
   if (cut)

@@ -39,3 +39,27 @@ def test_shares(torch_gpu, rest, m, empty):
     again = op.matmat(torch.from_numpy(V).cuda())
     ok = torch.from_numpy(full).cuda()
     assert torch.equal(Y[ok], again[ok])
+
+
+@pytest.mark.parametrize("chunk", [13.9, 14.0, 16.0, 17.9, 18.1])
+def test_entries_ahead(torch_gpu, chunk):
+    """Both sides of the rule for the entries loaded ahead (24 where a quad's chunk holds 14 to 18
+    on average), with chunks shorter than 16 and longer than 24 among them."""
+    torch = torch_gpu
+    from snapatac2_amd.tl._operator import SpectralOperator, _to_device_csr
+    rng = np.random.default_rng(int(10 * chunk))
+    n, m = 1500, 3000  # one block, three windows: 768 chunks
+    nnz = int(np.ceil(chunk * 768))
+    length = np.full(n, nnz // n)
+    length[rng.choice(n, nnz - length.sum(), replace=False)] += 1
+    cols = [np.sort(rng.choice(m, k, replace=False)) for k in length]
+    X = sp.csr_matrix((rng.integers(1, 200, nnz).astype(np.uint32), np.concatenate(cols),
+                       np.concatenate([[0], np.cumsum(length)])), shape=(n, m))
+    op = SpectralOperator(_to_device_csr(X, torch), layout="window")
+    w = op.window_csr
+    assert op.layout == "window" and w.n_blocks * w.n_windows == 3
+    V = rng.standard_normal((n, 16))
+    Xh, dinv, _, _ = osp.operator_parts(X)
+    ref = Xh @ (Xh.T @ V) - dinv[:, None] * V
+    Y = op.matmat(torch.from_numpy(V).cuda()).cpu().numpy()
+    assert np.abs(Y - ref).max() < 1e-5 * np.abs(ref).max()
