@@ -52,12 +52,6 @@ constexpr int64_t kChunkTarget = 65536;          // group-chunks that fill the c
 #define SNAPGPU_PANEL_INFLIGHT 8
 #endif
 constexpr int kInflight = SNAPGPU_PANEL_INFLIGHT;  // gathers in flight per lane
-#ifndef SNAPGPU_PANEL_INFLIGHT16
-#define SNAPGPU_PANEL_INFLIGHT16 16
-#endif
-// the same, 16-column packed-8 product: 16 against 8, per application of 3.9M entries
-// 117 and 142 us, of 130M 1.97 and 2.00 ms, of 820M (with windows) 13.53 and 13.64 ms
-constexpr int kInflight16 = SNAPGPU_PANEL_INFLIGHT16;
 static_assert(kPanel <= 32768, "the packed entry holds a 15-bit column");
 
 // Entries per group-chunk. A group streams its chunk alone, so a small matrix in
@@ -249,7 +243,11 @@ __global__ void chunk_kernel(const int64_t* __restrict__ pstart, const int64_t* 
 // adjoint of 20,000 cells x 100,000 features 1.25e-6 in one run of entries, 3.6e-7 so
 // ---------------------------------------------------------------------------
 constexpr int kSumBlock = 16;
-static_assert(kSumBlock % kInflight == 0 && kInflight16 == kSumBlock, "a step of gathers is (part of) one block");
+static_assert(kSumBlock % kInflight == 0, "a step of gathers is (part of) one block");
+// gathers in flight per lane of the 16-column packed-8 product: one block. 16 against 8, per
+// application of 3.9M entries 117 and 142 us, of 130M 1.97 and 2.00 ms, of 820M (with
+// windows) 13.53 and 13.64 ms
+constexpr int kInflight16 = kSumBlock;
 
 template <int MODE, bool FV>
 __device__ __forceinline__ float entry_value(uint32_t e, uint32_t v) {
