@@ -46,12 +46,11 @@ static bool region(std::string_view s, std::string_view* chrom, int64_t* start, 
   return true;
 }
 
+// Fibonacci hashing (Knuth, The Art of Computer Programming 6.4): the product with the
+// golden ratio's 64-bit fraction, its high half folded onto the low one.
 static uint64_t mix(uint64_t x) {
-  x ^= x >> 33;
-  x *= 0xff51afd7ed558ccdull;
-  x ^= x >> 33;
-  x *= 0xc4ceb9fe1a85ec53ull;
-  return x ^ (x >> 33);
+  x *= 0x9e3779b97f4a7c15ull;
+  return x ^ (x >> 32);
 }
 
 constexpr int kThreads = 256;
@@ -175,7 +174,7 @@ int snapgpu_region_parse(const char* h_text, int64_t n_bytes, int64_t n, const c
         next_id += at.second;
         last_id = at.first->second;
       }
-      size_t s = mix((uint64_t)a * 0x9e3779b97f4a7c15ull + mix((uint64_t)b + ((uint64_t)last_id << 40))) & (slots - 1);
+      size_t s = mix((uint64_t)a + mix((uint64_t)b + ((uint64_t)last_id << 40))) & (slots - 1);
       bool seen = false;
       for (; table[s] >= 0; s = (s + 1) & (slots - 1)) {
         const int64_t k = table[s];
