@@ -14,7 +14,9 @@ def _numpy(U, cols, scale):
     return out if scale is None else out * scale
 
 
-@pytest.mark.parametrize("n,k", [(1, 1), (7, 3), (1023, 32), (1024, 33), (1025, 31), (5000, 70)])
+# 256 rows per slice of the search, 64 slices at a time when their results are joined
+@pytest.mark.parametrize("n,k", [(1, 1), (7, 3), (255, 32), (256, 33), (257, 31), (1024, 2), (5000, 70), (16384, 3),
+                                 (16385, 2), (40000, 5)])
 @pytest.mark.parametrize("case", ["random", "ties", "zero", "nan", "strided"])
 def test_finish(torch_gpu, n, k, case):
     torch = torch_gpu
@@ -23,6 +25,8 @@ def test_finish(torch_gpu, n, k, case):
     U = rng.standard_normal((n, k + 2))
     if case == "ties":  # equal magnitudes of both signs, in many rows
         U = rng.integers(-2, 3, (n, k + 2)).astype(np.float64)
+        if n > 64 * 256:  # and the largest in two slices that one lane joins, 64 apart
+            U[200], U[64 * 256 + min(200, n - 64 * 256 - 1)] = (-5.0, 5.0) if k % 2 else (5.0, -5.0)
     if case == "zero":
         U[:, 0] = 0.0
     if case == "nan":
