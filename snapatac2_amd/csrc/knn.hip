@@ -70,7 +70,7 @@ enum Mode : int32_t { kModeFP32 = 0, kModeBF16 = 1 };
 // 1.02 * 192 * 2^-24 (|x||q| + |x|^2 / 2). All doubled by d^2 = |q|^2 - 2s, plus fp32
 // rounding of the inputs and of the norms: 2.4e-5 |x||q| + 1.3e-5 |x|^2 + 2e-6 |q|^2,
 // so c = 3e-5. (Two terms and three products leave 2^-15 |x||q|, which c = 4e-5 would
-// still cover; they send twice as many rows to the second tier.)
+// still cover; of a million clustered rows 515 then go to the second tier, and 418 so.)
 // FP32: 32 sequential FMAs (<= 32 * 2^-24), doubled, plus input rounding: c = 1e-5.
 constexpr double kEpsBF16 = 3.0e-5;
 constexpr double kEpsFP32 = 1.0e-5;
