@@ -575,7 +575,7 @@ static int launch(const Params& p, hipStream_t st) {
 // then repeated by the tile kernel above, which also takes bins so small that
 // such fragments are the rule (below kMinSegBin bases).
 //
-// Count and fill of 30,000 cells (209M fragments, bins of 500): 1.73 and 2.80 ms
+// Count and fill of 30,000 cells (209M fragments, bins of 500): 1.53 and 2.32 ms
 // against the tile kernel's 4.67 and 5.39, which merges every 64 fragments by
 // rank into a pending list.
 // ---------------------------------------------------------------------------
@@ -1019,7 +1019,7 @@ static int seg_launch(const Params& p, hipStream_t st) {
 }
 
 // Waves per cell: a cell's segments go side by side until the cells alone fill
-// the chip. 301 cells (2.1M fragments, the longest cell 60 thousand): 65 + 120 us
+// the chip. 301 cells (2.1M fragments, the longest cell 60 thousand): 72 + 113 us
 // with 16 waves per cell, where the tile kernel's one wave took 1886 + 2108.
 template <int STRATEGY, bool FILL, typename IdxT>
 static int seg_launch_waves(const Params& p, hipStream_t st) {
