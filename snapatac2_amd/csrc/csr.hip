@@ -195,6 +195,10 @@ static int col_window_sums(const int64_t* d_indptr, int64_t n, const IdxT* d_idx
   return SNAPGPU_OK;
 }
 
+// A kernel, not a memset: the call can be captured, and memset nodes have given wrong
+// results on replays after the first.
+__global__ void clear_kernel(unsigned long long* __restrict__ v) { *v = 0ull; }
+
 // out[j] = sums[j] as a double; *zeros += the sums that are not positive
 __global__ void __launch_bounds__(256) sums_f64_kernel(const int64_t* __restrict__ sums, int64_t m,
                                                        double* __restrict__ out, unsigned long long* __restrict__ zeros) {
@@ -249,7 +253,8 @@ int snapgpu_col_sums_f64(const int64_t* d_sums, int64_t m, double* d_out, uint64
   clear_error();
   SG_ARG(m >= 0 && d_zeros != nullptr && (m == 0 || (d_sums && d_out)), "bad arguments");
   hipStream_t st = as_stream(stream);
-  SG_HIP(hipMemsetAsync(d_zeros, 0, 8, st));
+  clear_kernel<<<1, 1, 0, st>>>(reinterpret_cast<unsigned long long*>(d_zeros));
+  SG_LAUNCH_CHECK();
   if (m == 0) return SNAPGPU_OK;
   sums_f64_kernel<<<(unsigned)std::min<int64_t>(ceil_div(m, 256), 2048), 256, 0, st>>>(
       d_sums, m, d_out, reinterpret_cast<unsigned long long*>(d_zeros));
